@@ -76,8 +76,10 @@ struct Stepper {
   template <class T>
   CBM_HD static T sqrt(T x) {
 #ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (sizeof(R) == 8 && sizeof(T) == 8)
-      return x == 0.0 || x == __builtin_inf() ? x : refined_root(x, __builtin_amdgcn_rsq(x));
+    if constexpr (sizeof(R) == 8 && sizeof(T) == 8) {
+      const T g = refined_root(x, __builtin_amdgcn_rsq(x));
+      return x == 0.0 || x == __builtin_inf() ? x : g;
+    }
 #endif
     return std::sqrt(x);
   }
@@ -466,77 +468,69 @@ struct Stepper {
   // 202-206).  The reference holds these coefficients in REAL(r_2) (FP64,
   // :36-38).  In FP32 (the mixed path) the sum -coef1 + sqrt(delcx) cancels
   // when coef1 > 0 and loses the root's digits, so there the equal
-  // 2 coef0 / (-coef1 - sqrt(delcx)) is taken, which keeps them: the
-  // canopy's GPP then stays as close to FP64 as the reference's own shipped
-  // build does.  FP64 keeps the reference's form.
-  CBM_HD static R larger_root(R coef2z, R coef1z, R coef0z, R delcxz) {
+  // 2 coef0 / (-coef1 - sqrt(delcx)) is taken, which keeps them: the canopy's
+  // GPP then stays as close to FP64 as the reference's own shipped build
+  // does.  FP64 keeps the reference's form.
+  CBM_HD static R larger_root(R coef2z, R coef1z, R coef0z) {
+    const R delcxz = p2(coef1z) - K(4.0) * coef0z * coef2z;
+    const R s = sqrt(MAX(K(0.0), delcxz));
     if constexpr (sizeof(R) == 4) {
-      if (coef1z > K(0.0)) return DIV(K(2.0) * coef0z, -coef1z - sqrt(MAX(K(0.0), delcxz)));
+      const bool b = coef1z > K(0.0);
+      const R d = (b ? -s : s) - coef1z;
+      return DIV(b ? K(2.0) * coef0z : d, b ? d : K(2.0) * coef2z);
     }
-    return DIV(-coef1z + sqrt(MAX(K(0.0), delcxz)), K(2.0) * coef2z);
+    const bool linear = fabs(coef2z) < K(1.0e-9);
+    return DIV(linear ? -coef0z : -coef1z + s, linear ? coef1z : K(2.0) * coef2z);
   }
 
-  // src/science/canopy/cbl_photosynthesis.F90:10-226, one leaf
+  // src/science/canopy/cbl_photosynthesis.F90:10-226, one leaf.  The three
+  // limits' quadratics are solved side by side, so that their chains of
+  // square roots and quotients overlap.  A coefficient of z^2 too small for
+  // the root (none with the shipped parameters) takes the reference's linear
+  // form: in FP64, whose one wave per SIMD waits on those chains, by selected
+  // operands of the one quotient, which keeps both leaves in one block (a
+  // day of 262,144 tiles 17.1 against 17.9 ms); in FP32, bound by issue, in
+  // a branch for the three (a day of 1,048,576 tiles 19.8 against 20.8 ms).
   CBM_HD static R photosynthesis_leaf(R csxz, R cx1z, R cx2z, R gswminz, R rdxz, R vcmxt3z,
                                           R vcmxt4z, R vx3z, R vx4z, R gs_coeffz, R fwsoilz) {
     const R effc4 = K(4000.0);
-    R coef0z, coef1z, coef2z, ciz, delcxz;
-    R anrubiscoz = K(0.0), anrubpz = K(0.0), ansinkz = K(0.0);
     R gf = DIV(gswminz * fwsoilz, RGSWC);
-    coef2z = gf + gs_coeffz * (vcmxt3z - (rdxz - vcmxt4z));
-    coef1z = (K(1.0) - csxz * gs_coeffz) * (vcmxt3z + vcmxt4z - rdxz) + DIV(gswminz * fwsoilz, RGSWC) * (cx1z - csxz) -
-             gs_coeffz * (vcmxt3z * cx2z / K(2.0) + cx1z * (rdxz - vcmxt4z));
-    coef0z = -(K(1.0) - csxz * gs_coeffz) * (vcmxt3z * cx2z / K(2.0) + cx1z * (rdxz - vcmxt4z)) -
-             DIV(gswminz * fwsoilz, RGSWC) * cx1z * csxz;
-    if (fabs(coef2z) > K(1.0e-9) && fabs(coef1z) < K(1.0e-9)) {
-      ciz = K(99999.0);
-      anrubiscoz = K(99999.0);
+    R coef0[3], coef1[3], coef2[3];
+    coef2[0] = gf + gs_coeffz * (vcmxt3z - (rdxz - vcmxt4z));
+    coef1[0] = (K(1.0) - csxz * gs_coeffz) * (vcmxt3z + vcmxt4z - rdxz) + DIV(gswminz * fwsoilz, RGSWC) * (cx1z - csxz) -
+               gs_coeffz * (vcmxt3z * cx2z / K(2.0) + cx1z * (rdxz - vcmxt4z));
+    coef0[0] = -(K(1.0) - csxz * gs_coeffz) * (vcmxt3z * cx2z / K(2.0) + cx1z * (rdxz - vcmxt4z)) -
+               DIV(gswminz * fwsoilz, RGSWC) * cx1z * csxz;
+    coef2[1] = gf + gs_coeffz * (vx3z - (rdxz - vx4z));
+    coef1[1] = (K(1.0) - csxz * gs_coeffz) * (vx3z + vx4z - rdxz) + DIV(gswminz * fwsoilz, RGSWC) * (cx2z - csxz) -
+               gs_coeffz * (vx3z * cx2z / K(2.0) + cx2z * (rdxz - vx4z));
+    coef0[1] = -(K(1.0) - csxz * gs_coeffz) * (vx3z * cx2z / K(2.0) + cx2z * (rdxz - vx4z)) -
+               DIV(gswminz * fwsoilz, RGSWC) * cx2z * csxz;
+    coef2[2] = gs_coeffz;
+    coef1[2] = gf + gs_coeffz * (rdxz - K(0.5) * vcmxt3z) + effc4 * vcmxt4z - gs_coeffz * csxz * effc4 * vcmxt4z;
+    coef0[2] = -DIV(gswminz * fwsoilz, RGSWC) * csxz * effc4 * vcmxt4z + DIV((rdxz - K(0.5) * vcmxt3z) * gswminz * fwsoilz, RGSWC);
+    R z[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) z[q] = larger_root(coef2[q], coef1[q], coef0[q]);
+    bool none[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+      none[q] = sizeof(R) == 8 && fabs(coef2[q]) < K(1.0e-9) && fabs(coef1[q]) < K(1.0e-9);
+    if (sizeof(R) == 4 && (fabs(coef2[0]) < K(1.0e-9) || fabs(coef2[1]) < K(1.0e-9) || fabs(coef2[2]) < K(1.0e-9))) {
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        if (fabs(coef2[q]) < K(1.0e-9)) {
+          z[q] = DIV(-coef0[q], coef1[q]);
+          none[q] = fabs(coef1[q]) < K(1.0e-9);
+        }
     }
-    if (fabs(coef2z) < K(1.e-9) && fabs(coef1z) >= K(1e-9)) {
-      ciz = DIV(-K(1.0) * coef0z, coef1z);
-      ciz = MAX(K(0.0), ciz);
-      anrubiscoz = DIV(vcmxt3z * (ciz - cx2z / K(2.0)), ciz + cx1z) + vcmxt4z - rdxz;
-    }
-    if (fabs(coef2z) >= K(1.e-9)) {
-      delcxz = p2(coef1z) - K(4.0) * coef0z * coef2z;
-      ciz = larger_root(coef2z, coef1z, coef0z, delcxz);
-      ciz = MAX(K(0.0), ciz);
-      anrubiscoz = DIV(vcmxt3z * (ciz - cx2z / K(2.0)), ciz + cx1z) + vcmxt4z - rdxz;
-    }
-    coef2z = gf + gs_coeffz * (vx3z - (rdxz - vx4z));
-    coef1z = (K(1.0) - csxz * gs_coeffz) * (vx3z + vx4z - rdxz) + DIV(gswminz * fwsoilz, RGSWC) * (cx2z - csxz) -
-             gs_coeffz * (vx3z * cx2z / K(2.0) + cx2z * (rdxz - vx4z));
-    coef0z = -(K(1.0) - csxz * gs_coeffz) * (vx3z * cx2z / K(2.0) + cx2z * (rdxz - vx4z)) -
-             DIV(gswminz * fwsoilz, RGSWC) * cx2z * csxz;
-    ciz = K(99999.0);
-    anrubpz = K(99999.0);
-    if (fabs(coef2z) < K(1.e-9) && fabs(coef1z) >= K(1.e-9)) {
-      ciz = DIV(-K(1.0) * coef0z, coef1z);
-      ciz = MAX(K(0.0), ciz);
-      anrubpz = DIV(vx3z * (ciz - cx2z / K(2.0)), ciz + cx2z) + vx4z - rdxz;
-    }
-    if (fabs(coef2z) >= K(1.e-9)) {
-      delcxz = p2(coef1z) - K(4.0) * coef0z * coef2z;
-      ciz = larger_root(coef2z, coef1z, coef0z, delcxz);
-      ciz = MAX(K(0.0), ciz);
-      anrubpz = DIV(vx3z * (ciz - cx2z / K(2.0)), ciz + cx2z) + vx4z - rdxz;
-    }
-    coef2z = gs_coeffz;
-    coef1z = gf + gs_coeffz * (rdxz - K(0.5) * vcmxt3z) + effc4 * vcmxt4z - gs_coeffz * csxz * effc4 * vcmxt4z;
-    coef0z = -DIV(gswminz * fwsoilz, RGSWC) * csxz * effc4 * vcmxt4z + DIV((rdxz - K(0.5) * vcmxt3z) * gswminz * fwsoilz, RGSWC);
-    if (fabs(coef2z) < K(1.0e-9) && fabs(coef1z) < K(1.0e-9)) {
-      ciz = K(99999.0);
-      ansinkz = K(99999.0);
-    }
-    if (fabs(coef2z) < K(1.e-9) && fabs(coef1z) >= K(1.e-9)) {
-      ciz = DIV(-K(1.0) * coef0z, coef1z);
-      ansinkz = ciz;
-    }
-    if (fabs(coef2z) >= K(1.e-9)) {
-      delcxz = p2(coef1z) - K(4.0) * coef0z * coef2z;
-      ciz = larger_root(coef2z, coef1z, coef0z, delcxz);
-      ansinkz = ciz;
-    }
+    R ciz = MAX(K(0.0), z[0]);
+    R anrubiscoz = DIV(vcmxt3z * (ciz - cx2z / K(2.0)), ciz + cx1z) + vcmxt4z - rdxz;
+    anrubiscoz = none[0] ? K(0.0) : anrubiscoz;
+    ciz = MAX(K(0.0), z[1]);
+    R anrubpz = DIV(vx3z * (ciz - cx2z / K(2.0)), ciz + cx2z) + vx4z - rdxz;
+    anrubpz = none[1] ? K(99999.0) : anrubpz;
+    const R ansinkz = none[2] ? K(99999.0) : z[2];
     return MIN(MIN(anrubiscoz, anrubpz), ansinkz);
   }
 
@@ -626,6 +620,7 @@ struct Stepper {
     const R tvair = t.met_tvair[0], tk = t.met_tk[0];
     const R fvl0 = t.rad_fvlai[0], fvl1 = t.rad_fvlai[1];
     const bool leaves = fvl0 + fvl1 > LAI_THRESH;
+    const bool c4 = PV(veg_frac4, 0) != K(0.0);
     // the reference's fixed count of 20 passes.  The hybrid polishes the
     // start of a sunlit leaf-bearing tile with a.max_passes passes and then
     // checks it by its leaf energy-balance residual: the leaf
@@ -641,6 +636,8 @@ struct Stepper {
     // NITER pass again from the reference's start instead was measured:
     // 0.547 against 0.523 ms per step at 1,048,576 tiles, and no more
     // accurate.)  Every other tile runs the reference's iteration.
+    // (one copy of the body: the hybrid's first passes would otherwise be
+    // peeled off, 8% more instructions)
     for (int k = 1; k <= 20; k++) {
       bool active = (vlaiw > LAI_THRESH && abs_deltlf > K(0.1));
       if constexpr (MODE == MODE_HYBRID) {
@@ -657,6 +654,7 @@ struct Stepper {
       // a tile that has converged keeps every value: the remaining passes of
       // the reference's fixed-count loop change nothing for it
       if (!active && k > 1) break;
+      anx[0] = anx[1] = K(0.0);
       if (active) {
         npass++;
         R tlfx = c.tlfx;
@@ -674,14 +672,6 @@ struct Stepper {
           ghr[l] = t.rad_gradis[l] + gh[l];
         }
         R frac4 = PV(veg_frac4, 0), vcmax = PV(veg_vcmax, 0);
-        R temp = xvcmxt3(tlfx) * vcmax * (K(1.0) - frac4);
-        vcmxt3[0] = t.rad_scalex[0] * temp;
-        vcmxt3[1] = t.rad_scalex[1] * temp;
-        temp = xvcmxt4(tlfx - TFRZ) * vcmax * frac4;
-        vcmxt4[0] = t.rad_scalex[0] * temp;
-        vcmxt4[1] = t.rad_scalex[1] * temp;
-        temp = xejmxt3(tlfx) * PV(veg_ejmax, 0) * (K(1.0) - frac4);
-        R ejmxt3_0 = t.rad_scalex[0] * temp, ejmxt3_1 = t.rad_scalex[1] * temp;
         R tdiff = tlfx - TREFK;
         R conkct = PV(veg_conkc0, 0) * exp(DIV(PV(veg_ekc, 0), RGAS * TREFK) * (K(1.0) - DIV(TREFK, tlfx)));
         R conkot = PV(veg_conko0, 0) * exp(DIV(PV(veg_eko, 0), RGAS * TREFK) * (K(1.0) - DIV(TREFK, tlfx)));
@@ -690,37 +680,54 @@ struct Stepper {
         cx2 = K(2.0) * GAM0 * (K(1.0) + GAM1 * tdiff + GAM2 * tdiff * tdiff);
         R alpha = PV(veg_alpha, 0), convex = PV(veg_convex, 0);
         R q0 = t.rad_qcan[0], q1 = t.rad_qcan[1];
-        vx3[0] = ej3x(q0 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_0);
-        vx3[1] = ej3x(q1 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_1);
-        vx4[0] = ej4x(q0 * jtomol * frac4, alpha, convex, vcmxt4[0]);
-        vx4[1] = ej4x(q1 * jtomol * frac4, alpha, convex, vcmxt4[1]);
+        // the C3 and the C4 terms each carry the class's share as a factor:
+        // without one they are zero, and their exponentials and roots are
+        // left out (in FP32 the C4 terms only: the branch around the C3 terms
+        // waits for the class table and costs more than it saves)
+        if (sizeof(R) == 4 || frac4 != K(1.0)) {
+          R temp = xvcmxt3(tlfx) * vcmax * (K(1.0) - frac4);
+          vcmxt3[0] = t.rad_scalex[0] * temp;
+          vcmxt3[1] = t.rad_scalex[1] * temp;
+          temp = xejmxt3(tlfx) * PV(veg_ejmax, 0) * (K(1.0) - frac4);
+          R ejmxt3_0 = t.rad_scalex[0] * temp, ejmxt3_1 = t.rad_scalex[1] * temp;
+          vx3[0] = ej3x(q0 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_0);
+          vx3[1] = ej3x(q1 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_1);
+        }
+        if (sizeof(R) == 4 ? c4 : frac4 != K(0.0)) {
+          R temp = xvcmxt4(tlfx - TFRZ) * vcmax * frac4;
+          vcmxt4[0] = t.rad_scalex[0] * temp;
+          vcmxt4[1] = t.rad_scalex[1] * temp;
+          vx4[0] = ej4x(q0 * jtomol * frac4, alpha, convex, vcmxt4[0]);
+          vx4[1] = ej4x(q1 * jtomol * frac4, alpha, convex, vcmxt4[1]);
+        }
         R cfrd = PV(veg_cfrd, 0);
         rdx[0] = (cfrd * vcmxt3[0] + cfrd * vcmxt4[0]);
         rdx[1] = (cfrd * vcmxt3[1] + cfrd * vcmxt4[1]);
         R a1 = DIV(PV(veg_a1gs, 0), K(1.0) + DIV(c.dsx, PV(veg_d0gs, 0)));
         gs_coeff[0] = DIV(fwsoil, c.csx[0] - K(0.0)) * a1;
         gs_coeff[1] = DIV(fwsoil, c.csx[1] - K(0.0)) * a1;
-      }
-      anx[0] = anx[1] = K(0.0);
-      if (active && leaves) {
-        if (fvl0 > LAI_THRESH)
-          anx[0] = photosynthesis_leaf(c.csx[0], cx1, cx2, gswmin[0], rdx[0], vcmxt3[0], vcmxt4[0], vx3[0],
-                                       vx4[0], gs_coeff[0], fwsoil);
-        if (fvl1 > LAI_THRESH)
-          anx[1] = photosynthesis_leaf(c.csx[1], cx1, cx2, gswmin[1], rdx[1], vcmxt3[1], vcmxt4[1], vx3[1],
-                                       vx4[1], gs_coeff[1], fwsoil);
-      }
-      if (active) {
-#pragma unroll
-        for (int l = 0; l < 2; l++) {
-          if (t.rad_fvlai[l] > LAI_THRESH) {
-            c.csx[l] = t.met_ca[0] - DIV(RGBWC * anx[l], c.gbhu[l] + c.gbhf[l]);
-            c.csx[l] = MAX(K(1.0e-4), c.csx[l]);
-            t.canopy_gswx[l] = MAX(K(1.e-3), gswmin[l] * fwsoil + MAX(K(0.0), RGSWC * gs_coeff[l] * anx[l]));
-            R gw = DIV(K(1.0), DIV(K(1.0), t.canopy_gswx[l]) + DIV(K(1.0), K(1.075) * (c.gbhu[l] + c.gbhf[l])));
-            gw = MAX(gw, K(0.00001));
-            psycst[l] = t.air_psyc[0] * DIV(ghr[l], gw);
-          }
+        // one leaf's assimilation, leaf-surface CO2 and conductances; `has`:
+        // the leaf class has leaves (else its values stay)
+        auto leaf = [&](int l, bool has) {
+          const R an = photosynthesis_leaf(c.csx[l], cx1, cx2, gswmin[l], rdx[l], vcmxt3[l], vcmxt4[l], vx3[l],
+                                           vx4[l], gs_coeff[l], fwsoil);
+          anx[l] = has && leaves ? an : K(0.0);
+          R cs = t.met_ca[0] - DIV(RGBWC * anx[l], c.gbhu[l] + c.gbhf[l]);
+          c.csx[l] = has ? MAX(K(1.0e-4), cs) : c.csx[l];
+          const R gsw = MAX(K(1.e-3), gswmin[l] * fwsoil + MAX(K(0.0), RGSWC * gs_coeff[l] * anx[l]));
+          t.canopy_gswx[l] = has ? gsw : t.canopy_gswx[l];
+          R gw = DIV(K(1.0), DIV(K(1.0), t.canopy_gswx[l]) + DIV(K(1.0), K(1.075) * (c.gbhu[l] + c.gbhf[l])));
+          gw = MAX(gw, K(0.00001));
+          const R ps = t.air_psyc[0] * DIV(ghr[l], gw);
+          psycst[l] = has ? ps : psycst[l];
+        };
+        // sunlit and shaded leaves side by side by day, shaded leaves alone
+        // without light
+        if (fvl0 > LAI_THRESH) {
+          leaf(0, true);
+          leaf(1, fvl1 > LAI_THRESH);
+        } else if (fvl1 > LAI_THRESH) {
+          leaf(1, true);
         }
         R dsatdk = t.air_dsatdk[0], dtv = tvair - tk;
         R cr = CAPP * RMAIR;
