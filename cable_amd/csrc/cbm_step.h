@@ -2065,7 +2065,7 @@ struct Stepper {
   // 725-729) and the balance accumulators (src/offline/cable_checks.F90
   // :472-618) in FP64
   CBM_HD void run() {
-    run([] {}, [] {});
+    run([] {}, [] {}, [] {});
   }
   // `late` runs after the canopy and before soil and snow: the resident
   // kernel loads there the state that only soil, snow, carbon and the
@@ -2073,8 +2073,9 @@ struct Stepper {
   // iteration.  `tail` runs after soil and snow, before the flux totals and
   // carbon: the resident kernel issues there the loads of the driver's
   // running sums, which sumcflux reads after the step.
-  template <class Late, class Tail>
-  CBM_HD void run(Late &&late, Tail &&tail) {
+  // `stash` runs before the canopy.
+  template <class Late, class Tail, class Stash>
+  CBM_HD void run(Late &&late, Tail &&tail, Stash &&stash) {
     R dels = (R)a.dels;
     if (a.driver) {
       // the offline driver before cbm, src/offline/cable_serial.F90:572-575
@@ -2097,6 +2098,7 @@ struct Stepper {
     t.rad_albedo_t[0] = (t.rad_albedo[0] + t.rad_albedo[1]) * K(0.5);
     t.ssnow_otss_0[0] = t.ssnow_otss[0];
     t.ssnow_otss[0] = t.ssnow_tss[0];
+    stash();
     define_canopy(sunlit_veg);
     late();
     t.ssnow_owetfac[0] = t.ssnow_wetfac[0];
