@@ -17,6 +17,7 @@
 #include <thread>
 #include <atomic>
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/cable_gpu.h"
 #include "cbm_kernel.h"
@@ -161,6 +162,7 @@ struct cable_gpu_ctx {
   int device = 0;
   // device position j holds the caller's tile order[j] (empty: identity)
   std::vector<int64_t> order;
+  uint32_t *d_order = nullptr;      // the same on the device, then its inverse ([2][mp]; null: identity)
   bool touched = false;             // device fields hold anything but zeros
   // ---- surrogate (mixed contexts) ----
   float *hyb = nullptr;             // [3][mp] previous-step leaf/canopy-air state
@@ -187,68 +189,87 @@ struct cable_gpu_ctx {
 namespace {
 // ---- batched transfers ----
 // One entry per field of a batched transfer: the field's device array, its
-// offset in the staging buffer and its length in 4-byte words.
+// offset in the staging buffer, its rows of mp values and a value's bytes.
 struct XferEntry {
   void *dev;
-  unsigned long long off, words;
+  unsigned long long off;
+  int rows, bytes;
 };
 constexpr size_t XFER_TABLE_BYTES = sizeof(XferEntry) * CABLE_NFIELDS;
 constexpr size_t XFER_ALIGN = 256;
 
-// stage -> fields (upload) or fields -> stage (download); blockIdx.y is the
-// entry, the x blocks stride over its words
-__global__ void xfer_kernel(const XferEntry *__restrict__ tab, uint32_t *__restrict__ stage, int to_fields) {
-  const XferEntry e = tab[blockIdx.y];
-  uint32_t *st = stage + e.off / 4, *dv = (uint32_t *)e.dev;
-  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < e.words;
-       i += (unsigned long long)gridDim.x * blockDim.x) {
-    if (to_fields)
-      dv[i] = st[i];
-    else
-      st[i] = dv[i];
+// dst(:, r) = src(perm, r)
+template <class T>
+__device__ inline void permute_rows(T *__restrict__ dst, const T *__restrict__ src,
+                                    const uint32_t *__restrict__ perm, int64_t mp, int rows) {
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < mp; t += (int64_t)gridDim.x * blockDim.x) {
+    const T *s = src + perm[t];
+    for (int r = 0; r < rows; r++) dst[r * mp + t] = s[r * mp];
   }
 }
 
-// host values of one field <-> its device-typed image in the staging
-// buffer, elements [i0, i1) (tile order and type conversion applied)
-void pack_range(const cable_gpu_ctx *c, const FieldMeta &f, const void *host, int ht, unsigned char *img, size_t i0,
-                size_t i1, bool to_device) {
-  const size_t de = dev_elem(f, c->precision), mp = (size_t)c->mp;
-  const int64_t *ord = c->order.empty() ? nullptr : c->order.data();
-  const bool same = (f.prec == 'I' && ht == CABLE_HOST_I32) || (f.prec != 'I' && de == 8 && ht == CABLE_HOST_F64) ||
-                    (f.prec != 'I' && de == 4 && ht == CABLE_HOST_F32);
-  if (same && !ord) {
-    if (to_device)
-      memcpy(img + i0 * de, (const unsigned char *)host + i0 * de, (i1 - i0) * de);
+// stage -> fields (upload) or fields -> stage (download); blockIdx.y is the
+// entry, the x blocks stride over its tiles.  The staging buffer holds the
+// caller's tile order: `perm` (null: the device's order is the caller's)
+// gives the source of each tile, so that the writes are contiguous and the
+// reads scattered within a row, which the caches hold.  Bound by those reads.
+// Ordering the tiles here rather than on the host, whose threads missed
+// their cache on every scattered value: the 11 surface fields of 1,048,576
+// tiles down in 2.2 ms (5.3 before), of 20,011 tiles with the soil in 0.28 ms
+// (0.46 before).
+__global__ void __launch_bounds__(256) xfer_kernel(const XferEntry *__restrict__ tab, unsigned char *stage,
+                                                   const uint32_t *__restrict__ perm, int64_t mp, int to_fields) {
+  const XferEntry e = tab[blockIdx.y];
+  void *dst = to_fields ? e.dev : stage + e.off;
+  const void *src = to_fields ? stage + e.off : e.dev;
+  if (perm) {
+    if (e.bytes == 8)
+      permute_rows((uint64_t *)dst, (const uint64_t *)src, perm, mp, e.rows);
     else
-      memcpy((unsigned char *)host + i0 * de, img + i0 * de, (i1 - i0) * de);
+      permute_rows((uint32_t *)dst, (const uint32_t *)src, perm, mp, e.rows);
     return;
   }
-  for (size_t i = i0; i < i1; i++) {
-    // rows of mp tiles; device position j of a row holds caller tile ord[j]
-    const size_t h = ord ? (i - i % mp) + (size_t)ord[i % mp] : i;
-    if (to_device) {
-      const double v = ht == CABLE_HOST_F64 ? ((const double *)host)[h]
-                       : ht == CABLE_HOST_F32 ? (double)((const float *)host)[h]
-                                              : (double)((const int32_t *)host)[h];
-      if (f.prec == 'I')
-        ((int32_t *)img)[i] = (int32_t)llround(v);
-      else if (de == 8)
-        ((double *)img)[i] = v;
-      else
-        ((float *)img)[i] = (float)v;
-    } else {
-      const double v = f.prec == 'I' ? (double)((const int32_t *)img)[i]
-                       : de == 8     ? ((const double *)img)[i]
-                                     : (double)((const float *)img)[i];
-      if (ht == CABLE_HOST_F64)
-        ((double *)host)[h] = v;
-      else if (ht == CABLE_HOST_F32)
-        ((float *)host)[h] = (float)v;
-      else
-        ((int32_t *)host)[h] = (int32_t)llround(v);
-    }
-  }
+  // both sides are aligned to 256 bytes: 16 bytes at a time, then the rest
+  const int64_t words = (int64_t)e.rows * mp * (e.bytes / 4), wide = words / 4;
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < wide; i += stride) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
+  for (int64_t i = 4 * wide + i0; i < words; i += stride) ((uint32_t *)dst)[i] = ((const uint32_t *)src)[i];
+}
+
+// n host values to or from their device-typed image
+template <class D, class S>
+void cast_range(D *dst, const S *src, size_t n) {
+  if constexpr (std::is_same<D, S>::value)
+    memcpy(dst, src, sizeof(D) * n);
+  else if constexpr (std::is_integral<D>::value)
+    for (size_t i = 0; i < n; i++) dst[i] = (D)llround((double)src[i]);
+  else
+    for (size_t i = 0; i < n; i++) dst[i] = (D)src[i];
+}
+template <class H>
+void pack_typed(const FieldMeta &f, size_t de, H *host, unsigned char *img, size_t i0, size_t n, bool to_device) {
+  auto move = [&](auto *dev) {
+    if (to_device)
+      cast_range(dev + i0, host + i0, n);
+    else
+      cast_range(host + i0, dev + i0, n);
+  };
+  if (f.prec == 'I') move((int32_t *)img);
+  else if (de == 8) move((double *)img);
+  else move((float *)img);
+}
+
+// host values of one field <-> its device-typed image in the staging
+// buffer, elements [i0, i1)
+void pack_range(const cable_gpu_ctx *c, const FieldMeta &f, void *host, int ht, unsigned char *img, size_t i0,
+                size_t i1, bool to_device) {
+  const size_t de = dev_elem(f, c->precision);
+  if (ht == CABLE_HOST_F64)
+    pack_typed(f, de, (double *)host, img, i0, i1 - i0, to_device);
+  else if (ht == CABLE_HOST_F32)
+    pack_typed(f, de, (float *)host, img, i0, i1 - i0, to_device);
+  else
+    pack_typed(f, de, (int32_t *)host, img, i0, i1 - i0, to_device);
 }
 
 int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts, const int *types, bool up);
@@ -260,24 +281,33 @@ size_t field_bytes(const cable_gpu_ctx *c, int id) {
 }
 
 // Several fields in one copy each way: the host side packs (unpacks) the
-// fields' device-typed images in the pinned staging buffer on up to eight
-// threads, one copy moves the buffer, one kernel scatters (gathers) the
-// fields on the device.  The transfer table rides in front of the upload's
+// fields' device-typed images in the pinned staging buffer, one copy moves
+// the buffer, one kernel scatters (gathers) the fields on the device and puts
+// the tiles in order.  The transfer table rides in front of the upload's
 // data; a download sends it ahead in a copy of its own.
+//
+// A small batch is moved by the kernel itself, on the pinned buffer: up to
+// XFER_DIRECT bytes the copies' latency is more than the kernel's reads and
+// writes over the bus take (11 fields down: 28 against 33 us at 77 tiles, 32
+// against 42 us at 1,200, 61 against 52 us at 4,000), half of that for an
+// upload that reads the pinned buffer in scattered order (36 against 39 us at
+// 700 tiles, 45 against 40 us at 1,200).  A thread packs each XFER_THREAD
+// bytes, up to eight: starting one costs as much as it saves below (11
+// fields of 8,000 tiles down: 67 us with one thread, 76 with three).
+constexpr size_t XFER_DIRECT = 128 << 10, XFER_THREAD = 1 << 20;
 int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts, const int *types, bool up) {
   const char *who = up ? "cable_gpu_upload_fields" : "cable_gpu_download_fields";
   if (n > CABLE_NFIELDS) return fail(CABLE_E_ARG, "%s: %d fields (at most %d)", who, n, CABLE_NFIELDS);
   std::vector<XferEntry> tab(n);
-  size_t off = XFER_TABLE_BYTES, maxw = 0;
+  size_t off = XFER_TABLE_BYTES;
   for (int k = 0; k < n; k++) {
     if (ids[k] < 0 || ids[k] >= CABLE_NFIELDS || !hosts[k])
       return fail(CABLE_E_ARG, "%s: bad field %d (entry %d)", who, ids[k], k);
     if (types[k] != CABLE_HOST_F64 && types[k] != CABLE_HOST_F32 && types[k] != CABLE_HOST_I32)
       return fail(CABLE_E_ARG, "%s: bad host type %d (entry %d)", who, types[k], k);
-    const size_t b = field_bytes(c, ids[k]);
-    tab[k] = {c->dev[ids[k]], off, b / 4};
-    maxw = std::max(maxw, (size_t)(b / 4));
-    off += (b + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN;
+    const FieldMeta &f = kFields[ids[k]];
+    tab[k] = {c->dev[ids[k]], off, f.n, (int)dev_elem(f, c->precision)};
+    off += (field_bytes(c, ids[k]) + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN;
   }
   if (n == 0) return CABLE_OK;
   if (off > c->stage_bytes) {
@@ -286,19 +316,19 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
     if (c->d_stage) HIPCHECK(hipFree(c->d_stage));
     c->h_stage = c->d_stage = nullptr;
     c->stage_bytes = 0;
-    HIPCHECK(hipHostMalloc((void **)&c->h_stage, off, hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void **)&c->h_stage, off, hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHECK(hipMalloc((void **)&c->d_stage, off));
     c->stage_bytes = off;
   }
   memcpy(c->h_stage, tab.data(), sizeof(XferEntry) * n);
-  // the fields cut in pieces of at most 4 Mi elements, shared out to threads
+  // the fields cut in pieces of at most 128 Ki elements, shared out to threads
   struct Piece {
     int k;
     size_t i0, i1;
   };
   std::vector<Piece> pieces;
   for (int k = 0; k < n; k++) {
-    const size_t cnt = (size_t)kFields[ids[k]].n * (size_t)c->mp, step = (size_t)1 << 22;
+    const size_t cnt = (size_t)kFields[ids[k]].n * (size_t)c->mp, step = (size_t)1 << 17;
     for (size_t i = 0; i < cnt; i += step) pieces.push_back({k, i, std::min(cnt, i + step)});
   }
   auto work = [&](bool to_device) {
@@ -310,31 +340,33 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
                    to_device);
       }
     };
-    const unsigned nt = (unsigned)std::min<size_t>({8, pieces.size(), std::max(1u, std::thread::hardware_concurrency())});
+    const unsigned nt = (unsigned)std::min<size_t>(
+        {8, pieces.size(), off / XFER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
     std::vector<std::thread> th;
     for (unsigned t = 1; t < nt; t++) th.emplace_back(run);
     run();
     for (auto &t : th) t.join();
   };
-  const dim3 grid((unsigned)std::min<size_t>(1024, (maxw + 255) / 256), (unsigned)n);
+    const uint32_t *perm = !c->d_order ? nullptr : up ? c->d_order : c->d_order + c->mp;
+  const bool direct = off <= (up && perm ? XFER_DIRECT / 2 : XFER_DIRECT);
+  unsigned char *stage = c->d_stage;
+  if (direct) HIPCHECK(hipHostGetDevicePointer((void **)&stage, c->h_stage, 0));
+  const dim3 grid((unsigned)std::min<int64_t>(1024, (c->mp + 255) / 256), (unsigned)n);
   if (up) {
     c->touched = true;
     work(true);
-    HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, off, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(xfer_kernel, grid, dim3(256), 0, c->stream, (const XferEntry *)c->d_stage,
-                       (uint32_t *)c->d_stage, 1);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(c->stream));
-  } else {
+    if (!direct) HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, off, hipMemcpyHostToDevice, c->stream));
+  } else if (!direct) {
     HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, sizeof(XferEntry) * n, hipMemcpyHostToDevice, c->stream));
-    hipLaunchKernelGGL(xfer_kernel, grid, dim3(256), 0, c->stream, (const XferEntry *)c->d_stage,
-                       (uint32_t *)c->d_stage, 0);
-    HIPCHECK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(xfer_kernel, grid, dim3(256), 0, c->stream, (const XferEntry *)stage, stage, perm, c->mp,
+                     up ? 1 : 0);
+  HIPCHECK(hipGetLastError());
+  if (!up && !direct)
     HIPCHECK(hipMemcpyAsync(c->h_stage + XFER_TABLE_BYTES, c->d_stage + XFER_TABLE_BYTES, off - XFER_TABLE_BYTES,
                             hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    work(false);
-  }
+  HIPCHECK(hipStreamSynchronize(c->stream));
+  if (!up) work(false);
   return CABLE_OK;
 }
 
@@ -492,7 +524,7 @@ int cable_gpu_destroy(cable_gpu_ctx *c) {
   if (c->d_stab) hipFree(c->d_stab);
   if (c->d_npass) hipFree(c->d_npass);
   void *sur[] = {c->cons_part, c->cons_acc, c->hyb, c->sx, c->sy, c->scount, c->sparams, c->snorm, c->pred, c->swt,
-                 c->nfallback, c->d_lit, c->d_litblk};
+                 c->nfallback, c->d_lit, c->d_litblk, c->d_order};
   for (void *p : sur)
     if (p) hipFree(p);
   if (c->h_stage) hipHostFree(c->h_stage);
@@ -675,6 +707,14 @@ int cable_gpu_set_tile_order(cable_gpu_ctx *c, const int64_t *order) {
     seen[(size_t)order[j]] = 1;
   }
   const std::vector<int64_t> old_order = c->order, new_order(order, order + c->mp);
+  std::vector<uint32_t> both(2 * (size_t)c->mp);
+  for (int64_t j = 0; j < c->mp; j++) {
+    both[(size_t)j] = (uint32_t)order[j];
+    both[(size_t)(c->mp + order[j])] = (uint32_t)j;
+  }
+  if (!c->d_order) HIPCHECK(hipMalloc((void **)&c->d_order, sizeof(uint32_t) * both.size()));
+  HIPCHECK(hipMemcpyAsync(c->d_order, both.data(), sizeof(uint32_t) * both.size(), hipMemcpyHostToDevice, c->stream));
+  HIPCHECK(hipStreamSynchronize(c->stream));
   if (!c->touched) {  // still zero-filled: nothing to carry over
     c->order = new_order;
     return CABLE_OK;
