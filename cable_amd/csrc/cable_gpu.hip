@@ -1105,17 +1105,20 @@ __device__ inline double synth_svp(double tk) {
 // a workgroup form them for all.  48 steps of 1,048,576 tiles: kernel
 // 2.5 -> 2.0 ms (32 B per tile-step at 0.8 TB/s), the call 7.7 -> 2.5 ms with the
 // gather off the host.
-constexpr int SYNTH_STEPS = 8;
+// Below SYNTH_TILES tiles a thread takes one step, or the eight in turn leave
+// the chip idle (the call at 256 tiles 26 against 48 us, at 16,384 75 against
+// 80 us; at 32,768 tiles 124 against 111 us).
+constexpr int SYNTH_STEPS = 8, SYNTH_TILES = 32768;
 template <class R>
 __global__ void __launch_bounds__(256)
-    synth_kernel(int64_t mp, int k_first, int nsteps, SynthKeys keys, double dels, double doy, double hod0,
+    synth_kernel(int64_t mp, int k_first, int nsteps, int per, SynthKeys keys, double dels, double doy, double hod0,
                  const uint32_t *__restrict__ order, const double *__restrict__ t0, const double *__restrict__ lat,
                  R *fsd1, R *fld, R *tk, R *qv, R *ua, R *pmb, R *precip, R *coszen) {
   const double two_pi = 2.0 * M_PI;
   const double pi_f = 3.1415927, d2r = pi_f / 180.0;  // sinbet's pi, src/params/cable_maths_constants_mod.F90:32
   __shared__ double diurnal_s[SYNTH_STEPS], swing_s[SYNTH_STEPS], hour_s[SYNTH_STEPS];
-  const int s0 = blockIdx.y * SYNTH_STEPS;
-  if (threadIdx.x < SYNTH_STEPS) {
+  const int s0 = blockIdx.y * per;
+  if ((int)threadIdx.x < per) {
     const double hod = hod0 + (double)(k_first + (int64_t)(s0 + (int)threadIdx.x)) * (dels / 3600.0);
     diurnal_s[threadIdx.x] = fmax(0.0, 1000.0 * sin(two_pi * (hod - 6.0) / 24.0));
     swing_s[threadIdx.x] = 5.0 * sin(two_pi * (hod - 9.0) / 24.0);
@@ -1128,7 +1131,7 @@ __global__ void __launch_bounds__(256)
   const double tmean = t0[t], xlat = lat[t];
   const double sindec = -sin(23.45 * d2r) * cos(2.0 * pi_f * (doy + 10.0) / 365.0);
   const double cz0 = sin(d2r * xlat) * sindec, cz1 = cos(d2r * xlat) * sqrt(1.0 - sindec * sindec);
-  for (int s = 0; s < SYNTH_STEPS && s0 + s < nsteps; s++) {
+  for (int s = 0; s < per && s0 + s < nsteps; s++) {
     const int64_t k = k_first + (int64_t)(s0 + s), o = (int64_t)(s0 + s) * mp + j;
     const double sw = diurnal_s[s] * (0.5 + 0.5 * synth_u(keys, 0, t, k));
     const double tair = tmean + swing_s[s];
@@ -1185,14 +1188,15 @@ int cable_gpu_synth_forcing(cable_gpu_ctx *c, int k_first, int nsteps, uint64_t 
   const double *d_t0 = (const double *)c->d_stage, *d_lat = d_t0 + mp;
   SynthKeys keys;
   for (int s = 0; s < NSYNTH; s++) keys.k[s] = mix64(mix64(seed) ^ (uint64_t)(s + 1));
-  const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)((nsteps + SYNTH_STEPS - 1) / SYNTH_STEPS));
+  const int per = mp >= SYNTH_TILES ? SYNTH_STEPS : 1;
+  const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)((nsteps + per - 1) / per));
   void **f = c->forc.data();
   if (c->precision == CABLE_PREC_MIXED)
-    hipLaunchKernelGGL(synth_kernel<float>, grid, dim3(256), 0, c->stream, c->mp, k_first, nsteps, keys, dels, doy,
+    hipLaunchKernelGGL(synth_kernel<float>, grid, dim3(256), 0, c->stream, c->mp, k_first, nsteps, per, keys, dels, doy,
                        hod0, c->d_order, d_t0, d_lat, (float *)f[0], (float *)f[1], (float *)f[2], (float *)f[3],
                        (float *)f[4], (float *)f[5], (float *)f[6], (float *)f[7]);
   else
-    hipLaunchKernelGGL(synth_kernel<double>, grid, dim3(256), 0, c->stream, c->mp, k_first, nsteps, keys, dels, doy,
+    hipLaunchKernelGGL(synth_kernel<double>, grid, dim3(256), 0, c->stream, c->mp, k_first, nsteps, per, keys, dels, doy,
                        hod0, c->d_order, d_t0, d_lat, (double *)f[0], (double *)f[1], (double *)f[2],
                        (double *)f[3], (double *)f[4], (double *)f[5], (double *)f[6], (double *)f[7]);
   HIPCHECK(hipGetLastError());
