@@ -916,7 +916,8 @@ struct Stepper {
   }
 
   // src/science/canopy/cable_canopy.F90:10-1048
-  CBM_HD void define_canopy(bool sunlit_veg) {
+  template <class Settled>
+  CBM_HD void define_canopy(bool sunlit_veg, Settled &&settled) {
     Can c;
     R dels = (R)a.dels;
     R vlaiw = t.canopy_vlaiw[0];
@@ -1018,6 +1019,7 @@ struct Stepper {
     t.canopy_fns_cor[0] = K(0.0);
     t.canopy_ga_cor[0] = K(0.0);
     radiation(sunlit_veg);
+    settled();
     // stability parameter of each NITER pass, kept in registers (zetar(:,1..4));
     // passes 1-3 set zeta1-zeta3 before passes 2-4 read them
     R zeta1 = ZETPOS + K(1), zeta2 = ZETA0, zeta3 = ZETA0;
@@ -2065,7 +2067,7 @@ struct Stepper {
   // 725-729) and the balance accumulators (src/offline/cable_checks.F90
   // :472-618) in FP64
   CBM_HD void run() {
-    run([] {}, [] {}, [] {});
+    run([] {}, [] {}, [] {}, [] {});
   }
   // `late` runs after the canopy and before soil and snow: the resident
   // kernel loads there the state that only soil, snow, carbon and the
@@ -2073,9 +2075,10 @@ struct Stepper {
   // iteration.  `tail` runs after soil and snow, before the flux totals and
   // carbon: the resident kernel issues there the loads of the driver's
   // running sums, which sumcflux reads after the step.
-  // `stash` runs before the canopy.
-  template <class Late, class Tail, class Stash>
-  CBM_HD void run(Late &&late, Tail &&tail, Stash &&stash) {
+  // `stash` runs before the canopy, `settled` in it before the leaf iteration,
+  // when the radiation, roughness and air diagnostics have their last values.
+  template <class Late, class Tail, class Stash, class Settled>
+  CBM_HD void run(Late &&late, Tail &&tail, Stash &&stash, Settled &&settled) {
     R dels = (R)a.dels;
     if (a.driver) {
       // the offline driver before cbm, src/offline/cable_serial.F90:572-575
@@ -2099,7 +2102,7 @@ struct Stepper {
     t.ssnow_otss_0[0] = t.ssnow_otss[0];
     t.ssnow_otss[0] = t.ssnow_tss[0];
     stash();
-    define_canopy(sunlit_veg);
+    define_canopy(sunlit_veg, settled);
     late();
     t.ssnow_owetfac[0] = t.ssnow_wetfac[0];
     soil_snow();
