@@ -184,6 +184,7 @@ struct cable_gpu_ctx {
   // twin ([transfer table | fields, each at a 256-byte offset]) ----
   unsigned char *h_stage = nullptr, *d_stage = nullptr;
   size_t stage_bytes = 0;
+  std::vector<hipEvent_t> xev;      // a download's copies, one each
 };
 
 namespace {
@@ -295,38 +296,139 @@ int ensure_stage(cable_gpu_ctx *c, size_t bytes) {
   return CABLE_OK;
 }
 
-// f(first, last) over pieces of 1 MiB of `bytes`, on a thread per MiB up to
-// eight
+// The staging buffer is packed (unpacked) in pieces on up to eight threads,
+// one per XFER_THREAD bytes (starting one costs as much as it saves below: 11
+// fields of 8,000 tiles down, 0.7 MB, 67 us with one thread, 76 with three),
+// and copied in units, each when its pieces are packed or before they are
+// unpacked, so that the copies and the host's work overlap: every field of
+// 49,149 tiles up in 3.9 ms (152 MB; 4.9 packed first), down in 2.9 ms (3.6).
+// Units of 1 and 2 MiB were slower (4.7 and 4.1 ms up), of 8 MiB faster for
+// this and slower for small batches.
+constexpr size_t XFER_THREAD = 1 << 20, XFER_PIECE = 512 << 10, XFER_UNIT = 4 << 20;
+
+// f(piece) for every piece of `bytes`
 template <class F>
-void parallel_pieces(size_t bytes, F &&f) {
-  const size_t step = (size_t)1 << 20;
+void on_threads(int device, size_t bytes, F &&f) {
+  const size_t pieces = (bytes + XFER_PIECE - 1) / XFER_PIECE;
   std::atomic<size_t> next(0);
   auto run = [&]() {
-    for (size_t b; (b = next.fetch_add(step)) < bytes;) f(b, std::min(bytes, b + step));
+    for (size_t q; (q = next.fetch_add(1)) < pieces;) f(q);
   };
-  const unsigned nt =
-      (unsigned)std::min<size_t>({8, bytes / step + 1, std::max(1u, std::thread::hardware_concurrency())});
+  const unsigned nt = (unsigned)std::min<size_t>(
+      {8, pieces, bytes / XFER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
   std::vector<std::thread> th;
-  for (unsigned t = 1; t < nt; t++) th.emplace_back(run);
+  for (unsigned t = 1; t < nt; t++) {
+    try {
+      th.emplace_back([&]() {
+        if (hipSetDevice(device) == hipSuccess) run();
+      });
+    } catch (...) {  // no more threads: those there do the work
+      break;
+    }
+  }
   run();
   for (auto &t : th) t.join();
 }
 
-// Several fields in one copy each way: the host side packs (unpacks) the
-// fields' device-typed images in the pinned staging buffer, one copy moves
-// the buffer, one kernel scatters (gathers) the fields on the device and puts
-// the tiles in order.  The transfer table rides in front of the upload's
-// data; a download sends it ahead in a copy of its own.
+// fill(b0, b1) packs bytes [b0, b1) of the staging buffer; `bytes` of it go
+// to its device twin (`copy`) on the context's stream
+template <class F>
+hipError_t stage_up(cable_gpu_ctx *c, size_t bytes, bool copy, F &&fill) {
+  constexpr size_t PER = XFER_UNIT / XFER_PIECE;
+  const size_t units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
+  std::vector<std::atomic<size_t>> packed(units);
+  for (auto &u : packed) u = 0;
+  std::atomic<int> err(hipSuccess);
+  on_threads(c->device, bytes, [&](size_t q) {
+    const size_t u = q / PER, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
+    fill(q * XFER_PIECE, std::min(bytes, (q + 1) * XFER_PIECE));
+    if (packed[u].fetch_add(1) + 1 == (u1 - u0 + XFER_PIECE - 1) / XFER_PIECE && copy) {
+      const hipError_t e = hipMemcpyAsync(c->d_stage + u0, c->h_stage + u0, u1 - u0, hipMemcpyHostToDevice, c->stream);
+      if (e != hipSuccess) err = e;
+    }
+  });
+  return (hipError_t)err.load();
+}
+
+// host arrays one after the other in the staging buffer, each at a multiple
+// of 256 bytes, and the same on the device
+struct StageList {
+  struct Seg {
+    const void *host;
+    size_t off, bytes;
+  };
+  std::vector<Seg> segs;
+  size_t bytes = 0;
+  // the array's offset
+  size_t add(const void *host, size_t n) {
+    const size_t off = bytes;
+    segs.push_back({host, off, n});
+    bytes += (n + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN;
+    return off;
+  }
+  hipError_t up(cable_gpu_ctx *c) const {
+    return stage_up(c, bytes, true, [&](size_t b0, size_t b1) {
+      for (const Seg &g : segs) {
+        const size_t l0 = std::max(b0, g.off), l1 = std::min(b1, g.off + g.bytes);
+        if (l0 < l1) memcpy(c->h_stage + l0, (const unsigned char *)g.host + (l0 - g.off), l1 - l0);
+      }
+    });
+  }
+};
+
+// the device twin's `bytes` come back (`copy`) on the context's stream and
+// drain(b0, b1) unpacks them; ends when all has arrived
+template <class F>
+hipError_t stage_down(cable_gpu_ctx *c, size_t bytes, bool copy, F &&drain) {
+  const size_t units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
+  hipError_t e = hipSuccess;
+  if (copy && units > 1) {
+    for (size_t u = 0; u < units && e == hipSuccess; u++) {
+      const size_t u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
+      if (c->xev.size() <= u) {
+        hipEvent_t ev;
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) c->xev.push_back(ev);
+      }
+      if (e == hipSuccess)
+        e = hipMemcpyAsync(c->h_stage + u0, c->d_stage + u0, u1 - u0, hipMemcpyDeviceToHost, c->stream);
+      if (e == hipSuccess) e = hipEventRecord(c->xev[u], c->stream);
+    }
+  } else {
+    if (copy) e = hipMemcpyAsync(c->h_stage, c->d_stage, bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  }
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);
+    return e;
+  }
+  std::atomic<int> err(hipSuccess);
+  on_threads(c->device, bytes, [&](size_t q) {
+    if (copy && units > 1) {
+      const hipError_t w = hipEventSynchronize(c->xev[q * XFER_PIECE / XFER_UNIT]);
+      if (w != hipSuccess) {
+        err = w;
+        return;
+      }
+    }
+    drain(q * XFER_PIECE, std::min(bytes, (q + 1) * XFER_PIECE));
+  });
+  return (hipError_t)err.load();
+}
+
+// Several fields in one transfer each way: the host side packs (unpacks) the
+// fields' device-typed images in the pinned staging buffer, one kernel
+// scatters (gathers) the fields on the device and puts the tiles in order.
+// The transfer table rides in front of the upload's data; a download sends it
+// ahead in a copy of its own.
 //
 // A small batch is moved by the kernel itself, on the pinned buffer: up to
 // XFER_DIRECT bytes the copies' latency is more than the kernel's reads and
 // writes over the bus take (11 fields down: 28 against 33 us at 77 tiles, 32
 // against 42 us at 1,200, 61 against 52 us at 4,000), half of that for an
 // upload that reads the pinned buffer in scattered order (36 against 39 us at
-// 700 tiles, 45 against 40 us at 1,200).  A thread packs each XFER_THREAD
-// bytes, up to eight: starting one costs as much as it saves below (11
-// fields of 8,000 tiles down: 67 us with one thread, 76 with three).
-constexpr size_t XFER_DIRECT = 128 << 10, XFER_THREAD = 1 << 20;
+// 700 tiles, 45 against 40 us at 1,200).
+constexpr size_t XFER_DIRECT = 128 << 10;
 int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts, const int *types, bool up) {
   const char *who = up ? "cable_gpu_upload_fields" : "cable_gpu_download_fields";
   if (n > CABLE_NFIELDS) return fail(CABLE_E_ARG, "%s: %d fields (at most %d)", who, n, CABLE_NFIELDS);
@@ -343,53 +445,48 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
   }
   if (n == 0) return CABLE_OK;
   if (const int r = ensure_stage(c, off)) return r;
-  memcpy(c->h_stage, tab.data(), sizeof(XferEntry) * n);
-  // the fields cut in pieces of at most 128 Ki elements, shared out to threads
-  struct Piece {
-    int k;
-    size_t i0, i1;
+  // bytes [b0, b1) of the staging buffer: the parts of the fields there
+  auto pack = [&](size_t b0, size_t b1, bool to_device) {
+    if (to_device && b0 < sizeof(XferEntry) * n) {
+      const size_t e = std::min(b1, sizeof(XferEntry) * n);
+      memcpy(c->h_stage + b0, (const unsigned char *)tab.data() + b0, e - b0);
+    }
+    int k = (int)(std::upper_bound(tab.begin(), tab.end(), b0,
+                                   [](size_t b, const XferEntry &e) { return b < e.off; }) - tab.begin());
+    for (k = std::max(0, k - 1); k < n && tab[k].off < b1; k++) {
+      const size_t de = (size_t)tab[k].bytes, cnt = (size_t)tab[k].rows * (size_t)c->mp;
+      const size_t i0 = b0 > tab[k].off ? std::min<size_t>(cnt, (b0 - tab[k].off) / de) : 0;
+      const size_t i1 = std::min<size_t>(cnt, (b1 - tab[k].off) / de);
+      if (i0 < i1)
+        pack_range(c, kFields[ids[k]], hosts[k], types[k], c->h_stage + tab[k].off, i0, i1, to_device);
+    }
   };
-  std::vector<Piece> pieces;
-  for (int k = 0; k < n; k++) {
-    const size_t cnt = (size_t)kFields[ids[k]].n * (size_t)c->mp, step = (size_t)1 << 17;
-    for (size_t i = 0; i < cnt; i += step) pieces.push_back({k, i, std::min(cnt, i + step)});
-  }
-  auto work = [&](bool to_device) {
-    std::atomic<size_t> next(0);
-    auto run = [&]() {
-      for (size_t q; (q = next.fetch_add(1)) < pieces.size();) {
-        const Piece &pc = pieces[q];
-        pack_range(c, kFields[ids[pc.k]], hosts[pc.k], types[pc.k], c->h_stage + tab[pc.k].off, pc.i0, pc.i1,
-                   to_device);
-      }
-    };
-    const unsigned nt = (unsigned)std::min<size_t>(
-        {8, pieces.size(), off / XFER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
-    std::vector<std::thread> th;
-    for (unsigned t = 1; t < nt; t++) th.emplace_back(run);
-    run();
-    for (auto &t : th) t.join();
-  };
-    const uint32_t *perm = !c->d_order ? nullptr : up ? c->d_order : c->d_order + c->mp;
+  const uint32_t *perm = !c->d_order ? nullptr : up ? c->d_order : c->d_order + c->mp;
   const bool direct = off <= (up && perm ? XFER_DIRECT / 2 : XFER_DIRECT);
   unsigned char *stage = c->d_stage;
   if (direct) HIPCHECK(hipHostGetDevicePointer((void **)&stage, c->h_stage, 0));
   const dim3 grid((unsigned)std::min<int64_t>(1024, (c->mp + 255) / 256), (unsigned)n);
   if (up) {
     c->touched = true;
-    work(true);
-    if (!direct) HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, off, hipMemcpyHostToDevice, c->stream));
-  } else if (!direct) {
-    HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, sizeof(XferEntry) * n, hipMemcpyHostToDevice, c->stream));
+    const hipError_t e = stage_up(c, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, true); });
+    if (e != hipSuccess) {
+      (void)hipStreamSynchronize(c->stream);
+      return fail(CABLE_E_HIP, "%s: %s", who, hipGetErrorString(e));
+    }
+  } else {
+    memcpy(c->h_stage, tab.data(), sizeof(XferEntry) * n);
+    if (!direct)
+      HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, sizeof(XferEntry) * n, hipMemcpyHostToDevice, c->stream));
   }
   hipLaunchKernelGGL(xfer_kernel, grid, dim3(256), 0, c->stream, (const XferEntry *)stage, stage, perm, c->mp,
                      up ? 1 : 0);
   HIPCHECK(hipGetLastError());
-  if (!up && !direct)
-    HIPCHECK(hipMemcpyAsync(c->h_stage + XFER_TABLE_BYTES, c->d_stage + XFER_TABLE_BYTES, off - XFER_TABLE_BYTES,
-                            hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
-  if (!up) work(false);
+  if (up) {
+    HIPCHECK(hipStreamSynchronize(c->stream));
+  } else {
+    const hipError_t e = stage_down(c, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, false); });
+    if (e != hipSuccess) return fail(CABLE_E_HIP, "%s: %s", who, hipGetErrorString(e));
+  }
   return CABLE_OK;
 }
 
@@ -555,6 +652,7 @@ int cable_gpu_destroy(cable_gpu_ctx *c) {
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
   for (hipEvent_t ev : c->kev) hipEventDestroy(ev);
+  for (hipEvent_t ev : c->xev) hipEventDestroy(ev);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return CABLE_OK;
@@ -932,9 +1030,13 @@ __device__ inline R met_svp(R tk) {
   return pow(R(10.0), ewlog4);
 }
 
+// (12 steps of 131,071 tiles: 1.2 ms, 2.1 ms in 13 buffers allocated and
+// copied one by one from pageable memory)
+constexpr size_t MET_STAGE = 64 << 20;
+
 struct MetArgs {
   const float *swdown, *lwdown, *tair, *qair, *wind, *wind_e, *psurf, *rainf;
-  const int64_t *tix;       // device position -> caller tile
+  const uint32_t *order;    // device position -> caller tile (null: the same)
   const double *elev, *lat; // per caller tile
   const double *hod, *doy;  // per step of the window
   double tair_offset, psurf_scale, rainf_scale;
@@ -954,7 +1056,7 @@ __global__ void __launch_bounds__(256) met_kernel(int64_t mp, MetArgs m, R *fsd1
                                                   R *pmb, R *precip, R *coszen) {
   const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (j >= mp) return;
-  const int64_t t = m.tix[j], k = blockIdx.y, src = k * mp + t, o = k * mp + j;
+  const int64_t t = m.order ? (int64_t)m.order[j] : j, k = blockIdx.y, src = k * mp + t, o = k * mp + j;
   const R tair = (R)m.tair[src] + (R)m.tair_offset;
   R ps;
   if (m.psurf) {
@@ -1174,18 +1276,16 @@ int cable_gpu_synth_forcing(cable_gpu_ctx *c, int k_first, int nsteps, uint64_t 
   }
   // the per-tile inputs through the staging buffer, in the caller's order
   // (the draws are keyed by the caller's tile)
-  int r = ensure_stage(c, 2 * sizeof(double) * mp);
-  if (r) return r;
-  parallel_pieces(2 * sizeof(double) * mp, [&](size_t b0, size_t b1) {
-    const size_t half = sizeof(double) * mp;
-    if (b0 < half) memcpy(c->h_stage + b0, (const unsigned char *)t0 + b0, std::min(b1, half) - b0);
-    if (b1 > half) {
-      const size_t l0 = std::max(b0, half);
-      memcpy(c->h_stage + l0, (const unsigned char *)lat + (l0 - half), b1 - l0);
-    }
-  });
-  HIPCHECK(hipMemcpyAsync(c->d_stage, c->h_stage, 2 * sizeof(double) * mp, hipMemcpyHostToDevice, c->stream));
-  const double *d_t0 = (const double *)c->d_stage, *d_lat = d_t0 + mp;
+  StageList in;
+  in.add(t0, sizeof(double) * mp);
+  const size_t lat_off = in.add(lat, sizeof(double) * mp);
+  if (const int r = ensure_stage(c, in.bytes)) return r;
+  const hipError_t e = in.up(c);
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(c->stream);
+    return fail(CABLE_E_HIP, "cable_gpu_synth_forcing: %s", hipGetErrorString(e));
+  }
+  const double *d_t0 = (const double *)c->d_stage, *d_lat = (const double *)(c->d_stage + lat_off);
   SynthKeys keys;
   for (int s = 0; s < NSYNTH; s++) keys.k[s] = mix64(mix64(seed) ^ (uint64_t)(s + 1));
   const int per = mp >= SYNTH_TILES ? SYNTH_STEPS : 1;
@@ -1236,58 +1336,47 @@ int cable_gpu_set_met(cable_gpu_ctx *c, int k_first, int nsteps, double dels, co
     c->nsteps_forc = 0;
     for (int i = 0; i < 8; i++) HIPCHECK(hipMalloc(&c->forc[i], bytes));
   }
-  // inputs to the device: the met variables in the caller's tile order
-  std::vector<void *> tmp;
-  auto up = [&](const void *h, size_t nb) -> void * {
-    if (!h) return nullptr;
-    void *d = nullptr;
-    if (hipMalloc(&d, nb) != hipSuccess) return nullptr;
-    tmp.push_back(d);
-    if (hipMemcpyAsync(d, h, nb, hipMemcpyHostToDevice, c->stream) != hipSuccess) return nullptr;
-    return d;
-  };
-  std::vector<int64_t> tix(mp);
-  for (size_t j = 0; j < mp; j++) tix[j] = c->order.empty() ? (int64_t)j : c->order[j];
-  MetArgs a;
-  memset(&a, 0, sizeof a);
-  const size_t fb = sizeof(float) * n;
-  a.swdown = (const float *)up(m->swdown, fb);
-  a.lwdown = (const float *)up(m->lwdown, fb);
-  a.tair = (const float *)up(m->tair, fb);
-  a.qair = (const float *)up(m->qair, fb);
-  a.wind = (const float *)up(m->wind, fb);
-  a.wind_e = (const float *)up(m->wind_e, fb);
-  a.psurf = (const float *)up(m->psurf, fb);
-  a.rainf = (const float *)up(m->rainf, fb);
-  a.tix = (const int64_t *)up(tix.data(), sizeof(int64_t) * mp);
-  a.elev = (const double *)up(m->elevation, sizeof(double) * mp);
-  a.lat = (const double *)up(m->latitude, sizeof(double) * mp);
-  a.hod = (const double *)up(hod.data(), sizeof(double) * hod.size());
-  a.doy = (const double *)up(doy.data(), sizeof(double) * doy.size());
-  a.tair_offset = m->tair_offset;
-  a.psurf_scale = m->psurf_scale;
-  a.rainf_scale = m->rainf_scale;
-  a.qair_is_rh = m->qair_is_rh;
-  const bool ok = a.swdown && a.tair && a.qair && a.wind && a.rainf && a.tix && a.lat && a.hod && a.doy &&
-                  (!m->lwdown || a.lwdown) && (!m->wind_e || a.wind_e) && (!m->psurf || a.psurf) &&
-                  (!m->elevation || a.elev);
-  hipError_t e = hipSuccess;
-  if (ok) {
-    const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)nsteps);
-    void **f = c->forc.data();
-    if (c->precision == CABLE_PREC_MIXED)
-      hipLaunchKernelGGL(met_kernel<float>, grid, dim3(256), 0, c->stream, c->mp, a, (float *)f[0], (float *)f[1],
-                         (float *)f[2], (float *)f[3], (float *)f[4], (float *)f[5], (float *)f[6], (float *)f[7]);
-    else
-      hipLaunchKernelGGL(met_kernel<double>, grid, dim3(256), 0, c->stream, c->mp, a, (double *)f[0], (double *)f[1],
-                         (double *)f[2], (double *)f[3], (double *)f[4], (double *)f[5], (double *)f[6],
-                         (double *)f[7]);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  // the met variables to the device in the caller's tile order, through the
+  // staging buffer: as many steps at a time as MET_STAGE bytes hold
+  const float *const vars[8] = {m->swdown, m->lwdown, m->tair, m->qair, m->wind, m->wind_e, m->psurf, m->rainf};
+  size_t per_step = 0;
+  for (const float *v : vars) per_step += v ? sizeof(float) * mp : 0;
+  const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)nsteps, MET_STAGE / per_step));
+  for (int s0 = 0; s0 < nsteps; s0 += chunk) {
+    const int ns = std::min(chunk, nsteps - s0);
+    StageList in;
+    const size_t lat = in.add(m->latitude, sizeof(double) * mp);
+    const size_t elev = m->elevation ? in.add(m->elevation, sizeof(double) * mp) : 0;
+    const size_t hods = in.add(hod.data() + s0, sizeof(double) * (size_t)ns);
+    const size_t doys = in.add(doy.data() + s0, sizeof(double) * (size_t)ns);
+    size_t at[8];
+    for (int v = 0; v < 8; v++)
+      at[v] = vars[v] ? in.add(vars[v] + (size_t)s0 * mp, sizeof(float) * (size_t)ns * mp) : 0;
+    if (const int r = ensure_stage(c, in.bytes)) return r;
+    hipError_t e = in.up(c);
+    auto var = [&](int v) { return vars[v] ? (const float *)(c->d_stage + at[v]) : nullptr; };
+    const MetArgs a = {var(0), var(1), var(2), var(3), var(4), var(5), var(6), var(7), c->d_order,
+                       m->elevation ? (const double *)(c->d_stage + elev) : nullptr,
+                       (const double *)(c->d_stage + lat), (const double *)(c->d_stage + hods),
+                       (const double *)(c->d_stage + doys), m->tair_offset, m->psurf_scale, m->rainf_scale,
+                       m->qair_is_rh};
+    const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)ns);
+    auto go = [&](auto zero) {
+      using R = decltype(zero);
+      R *f[8];
+      for (int i = 0; i < 8; i++) f[i] = (R *)c->forc[i] + (size_t)s0 * mp;
+      hipLaunchKernelGGL(met_kernel<R>, grid, dim3(256), 0, c->stream, c->mp, a, f[0], f[1], f[2], f[3], f[4], f[5],
+                         f[6], f[7]);
+    };
+    if (e == hipSuccess) {
+      if (c->precision == CABLE_PREC_MIXED) go(0.0f);
+      else go(0.0);
+      e = hipGetLastError();
+    }
+    const hipError_t w = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = w;
+    if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString(e));
   }
-  for (void *d : tmp) hipFree(d);
-  if (!ok) return fail(CABLE_E_HIP, "cable_gpu_set_met: device buffers for the met variables");
-  if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString(e));
   const int ids[8] = {CABLE_F_met_fsd, CABLE_F_met_fld, CABLE_F_met_tk, CABLE_F_met_qv,
                       CABLE_F_met_ua, CABLE_F_met_pmb, CABLE_F_met_precip, CABLE_F_met_coszen};
   std::vector<void *> tab = c->dev;
