@@ -216,13 +216,19 @@ struct TileOut {
 // without a register held or a second wait for memory: reading it after the
 // canopy from memory left both waves of a SIMD (FP64: its one wave) waiting.
 // A day of 1,048,576 tiles in mixed precision 19.8 -> 18.9 ms, of 262,144 in
-// FP64 17.0 -> 16.8 ms.  55 KB of a 256-lane workgroup's LDS in FP32, 20 KB
-// of a wave's in FP64: with the tables, two and four workgroups per CU fit
-// the 160 KB.  A lane's values are LANES apart.
+// FP64 17.0 -> 16.8 ms.  The driver's carbon sums, which only the step's end
+// reads, come the same way, and what radiation leaves for soil, snow and the
+// balances and the leaf iteration does not read (PARK0 on) waits there rather
+// than in scratch memory: scratch instructions 72 -> 38 (FP64) and 33 -> 27,
+// 262,144 tiles 16.3 -> 15.9 ms, 1,048,576 mixed 18.8 -> 18.5 ms.  73 KB of a
+// 256-lane workgroup's LDS in FP32, 31 KB of a wave's in FP64: with the
+// tables, two and four workgroups per CU fit the 160 KB.  A lane's values are
+// LANES apart.
 template <class R>
 struct LateStage {
   static constexpr int LANES = sizeof(R) == 8 ? 64 : 256;  // the kernel's workgroup
-  static constexpr int NF = sizeof(R) == 8 ? 21 : 18, ND = 18;
+  // default REAL values (the carbon sums from SUM0, the parked values from PARK0), FP64 values
+  static constexpr int SUM0 = 18, PARK0 = SUM0 + 9, NF = PARK0 + (sizeof(R) == 8 ? 16 : 8), ND = 18;
   typename DevT<R, 'F'>::type *f = nullptr;
   double *d = nullptr;
 };
@@ -299,7 +305,7 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
   FieldTable F = (FieldTable)(uintptr_t)a.F;
   Tile<R> T;
   // (STAGE) the late state on its way to LDS
-  typename DevT<R, 'F'>::type lf[LateStage<R>::NF];
+  typename DevT<R, 'F'>::type lf[LateStage<R>::PARK0];
   double ld_[LateStage<R>::ND];
   // ---- gather ----
   if constexpr (FULL) {
@@ -380,13 +386,11 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
       LD_(ssnow_wb, 1, 6) LD_(ssnow_wbice, 1, 6) LD_(drv_owb, 0, 1) LD_(bal_ebal_tot, 0, 1) LD_(bal_wbal_tot, 0, 1)
       LD_(bal_precip_tot, 0, 1) LD_(bal_rnoff_tot, 0, 1) LD_(bal_evap_tot, 0, 1) LD_(bal_radbalsum, 0, 1)
       LD_(ssnow_gammzz, 0, 1)
+      LF_(sum_flux_sumpn, 0, 1) LF_(sum_flux_sumrp, 0, 1) LF_(sum_flux_sumrpw, 0, 1) LF_(sum_flux_sumrpr, 0, 1)
+      LF_(sum_flux_sumrs, 0, 1) LF_(sum_flux_sumrd, 0, 1) LF_(sum_flux_dsumpn, 0, 1) LF_(sum_flux_dsumrp, 0, 1)
+      LF_(sum_flux_dsumrd, 0, 1)
 #undef LF_
 #undef LD_
-      if constexpr (sizeof(R) == 8) {
-        lf[n++] = T.met_fsd[0];
-        lf[n++] = T.met_precip[0];
-        lf[n++] = T.ssnow_tss[0];
-      }
     }
 #undef LDS_
 #undef LDD_
@@ -414,7 +418,33 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
 #undef X
     }
   };
-  auto settled = [&]() { written(std::integral_constant<int, FIELD_SETTLED>{}); };
+  // (STAGE) values that the leaf iteration does not read, in LDS through it
+  auto parked = [&](auto &&move) {
+    int n = LateStage<R>::PARK0;
+    move(T.ssnow_wbtot1[0], n++);
+    move(T.ssnow_wbtot2[0], n++);
+    move(T.ssnow_wb_lake[0], n++);
+    move(T.ssnow_snage[0], n++);
+    move(T.ssnow_ssdnn[0], n++);
+    move(T.rad_albedo[0], n++);
+    move(T.rad_albedo[1], n++);
+    move(T.veg_vlai[0], n++);
+    if constexpr (sizeof(R) == 8) {
+      move(T.met_fsd[0], n++);
+      move(T.met_fsd[1], n++);
+      move(T.met_precip[0], n++);
+      move(T.met_precip_sn[0], n++);
+      move(T.ssnow_otss[0], n++);
+      move(T.rad_qcan[2], n++);
+      move(T.rad_qcan[3], n++);
+      move(T.rad_flws[0], n++);
+    }
+  };
+  auto unpark = [&]() { parked([&](R &x, int n) { x = late_lds.f[LateStage<R>::LANES * n]; }); };
+  auto settled = [&]() {
+    written(std::integral_constant<int, FIELD_SETTLED>{});
+    if constexpr (STAGE) parked([&](R &x, int n) { late_lds.f[LateStage<R>::LANES * n] = x; });
+  };
   auto late = [&]() {
     if constexpr (FULL) {
       __asm__ __volatile__("" ::: "memory");  // fresh reads, as below
@@ -449,14 +479,7 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
         LD_(ssnow_gammzz, 0, 1)
 #undef LF_
 #undef LD_
-        if constexpr (sizeof(R) == 8) {
-          const R fsd = late_lds.f[LateStage<R>::LANES * n++], pr = late_lds.f[LateStage<R>::LANES * n++];
-          T.met_fsd[0] = fsd;
-          T.met_fsd[1] = fsd;
-          T.met_precip[0] = pr;
-          T.met_precip_sn[0] = (T.met_tk[0] <= R(273.16)) ? pr : R(0.0);
-          T.ssnow_otss[0] = late_lds.f[LateStage<R>::LANES * n++];
-        }
+        unpark();
         return;
       }
 #define LDL_(T_, id, k0, n) \
@@ -495,7 +518,12 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
   // the offline driver's running carbon sums (driver mode): the resident
   // run reads the previous step's sums only after soil and snow
   auto tail = [&]() {
-    if constexpr (!FULL) {
+    if constexpr (STAGE) {  // (every resident step is the driver's)
+      int n = LateStage<R>::SUM0;
+      for (R *x : {T.sum_flux_sumpn, T.sum_flux_sumrp, T.sum_flux_sumrpw, T.sum_flux_sumrpr, T.sum_flux_sumrs,
+                   T.sum_flux_sumrd, T.sum_flux_dsumpn, T.sum_flux_dsumrp, T.sum_flux_dsumrd})
+        *x = late_lds.f[LateStage<R>::LANES * n++];
+    } else if constexpr (!FULL) {
       if (a.driver) {
           using DT = typename DevT<R, 'F'>::type;
         __asm__ __volatile__("" ::: "memory");
@@ -510,7 +538,7 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
   auto stash = [&]() {
     if constexpr (STAGE) {
 #pragma unroll
-      for (int q = 0; q < LateStage<R>::NF; q++) late_lds.f[LateStage<R>::LANES * q] = lf[q];
+      for (int q = 0; q < LateStage<R>::PARK0; q++) late_lds.f[LateStage<R>::LANES * q] = lf[q];
 #pragma unroll
       for (int q = 0; q < LateStage<R>::ND; q++) late_lds.d[LateStage<R>::LANES * q] = ld_[q];
     }
@@ -535,7 +563,13 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
   }
   // ---- scatter ----
 #ifdef __HIP_DEVICE_COMPILE__
-  if constexpr (!FULL) asm volatile("" : "+s"(F));  // the pointers are read again, not held
+  if constexpr (!FULL) {
+    asm volatile("" : "+s"(F));  // the pointers are read again, not held
+    // the lane offset formed here, so that the stores add it themselves
+    uint32_t t32 = (uint32_t)t;
+    asm volatile("" : "+v"(t32));
+    t = t32;
+  }
 #endif
   if constexpr (FULL) {
     written(std::integral_constant<int, 0>{});
