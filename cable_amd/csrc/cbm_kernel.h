@@ -138,8 +138,8 @@ CBM_HD void load_feature_raw(const StepArgs &a, const FeatureSrc &p, int64_t t, 
 }
 
 // vrow, srow: the rows of the tile's vegetation type and soil type
-template <class R>
-CBM_HD void finish_features(const StepArgs &a, const FeatureRaw<R> &r, const double *vrow, const double *srow,
+template <class R, class V>
+CBM_HD void finish_features(const StepArgs &a, const FeatureRaw<R> &r, const V *vrow, const double *srow,
                             float *x) {
   const float tk = (float)r.tk, qv = (float)r.qv;
   const float vlai = r.iveg >= 14 ? 0.0f : (float)r.vlai;
@@ -181,8 +181,8 @@ CBM_HD void finish_features(const StepArgs &a, const FeatureRaw<R> &r, const dou
   x[23] = (float)r.rtsoil;
 }
 
-template <class R>
-CBM_HD void surrogate_features(const StepArgs &a, int64_t t, const double *vrow, const double *srow, float *x) {
+template <class R, class V>
+CBM_HD void surrogate_features(const StepArgs &a, int64_t t, const V *vrow, const double *srow, float *x) {
   FeatureRaw<R> r;
   load_feature_raw<R>(a, feature_src(a), t, r);
   finish_features<R>(a, r, vrow, srow, x);
@@ -298,9 +298,12 @@ constexpr int field_phase(int id) {
 // the results.  vtab/stab are the class tables (TABLES), staged in LDS by the
 // kernel.  Host and device code: the test suite also runs it on the CPU, on
 // host arrays, under the sanitizers.
-template <class R, bool FULL, bool TABLES, int MODE, bool CONS, bool STAGE = false>
-CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const double *stab,
-                      TileOut<MODE, CONS> &o, LateStage<R> late_lds = {}) {
+// xtab: the derived columns (STAGE); vdtab/sdtab: FP64 columns beside an FP32
+// table (ClassRows).
+template <class R, bool FULL, bool TABLES, int MODE, bool CONS, bool STAGE = false, class V = double>
+CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> *vtab,
+                      const std::common_type_t<V> *stab, TileOut<MODE, CONS> &o, LateStage<R> late_lds = {},
+                      const V *xtab = nullptr, const double *vdtab = nullptr, const double *sdtab = nullptr) {
   const int64_t mp = a.mp;
   FieldTable F = (FieldTable)(uintptr_t)a.F;
   Tile<R> T;
@@ -396,9 +399,18 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
 #undef LDD_
   }
   const int iv = T.veg_iveg[0] - 1, is = T.soil_isoilm[0] - 1;
-  const double *vrow = TABLES ? vtab + (iv < 0 ? 0 : iv) * VC_N : nullptr;
-  const double *srow = TABLES ? stab + (is < 0 ? 0 : is) * SC_N : nullptr;
-  Stepper<R, FULL, TABLES, MODE> S(T, a, vrow, srow);
+  ClassRows<V> rows;
+  if constexpr (TABLES) {
+    const int v = iv < 0 ? 0 : iv, s = is < 0 ? 0 : is;
+    rows.v = vtab + v * VC_N;
+    rows.s = stab + s * SC_N;
+    if constexpr (STAGE) rows.x = xtab + v * VX_N;
+    if constexpr (sizeof(V) == 4) {
+      rows.vd = vdtab + v * NVEGD;
+      rows.sd = sdtab + s * SC_N;
+    }
+  }
+  Stepper<R, FULL, TABLES, MODE, V, STAGE> S(T, a, rows);
   // FULL: the fields of a phase written
   auto written = [&](auto phase) {
     if constexpr (FULL) {
@@ -508,7 +520,12 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
 #undef LDD_
     }
   };
-  if constexpr (MODE == MODE_CAPTURE) surrogate_features<R>(a, t, vrow, srow, o.feat);
+  if constexpr (MODE == MODE_CAPTURE) {
+    const double *sd;
+    if constexpr (sizeof(V) == 4) sd = rows.sd;
+    else sd = rows.s;
+    surrogate_features<R>(a, t, rows.v, sd, o.feat);
+  }
   if constexpr (MODE == MODE_HYBRID) {
     if (a.pred) {
 #pragma unroll
@@ -613,15 +630,20 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const double *vtab, const do
 template <class R, bool FULL, bool TABLES, int MODE = MODE_PLAIN, bool CONS = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 2 : 1, sizeof(R) == 4 ? 2 : 1)))
 cbm_kernel(StepArgs a) {
-  __shared__ double lds_v[TABLES ? NVEGCLASS * VC_N : 1];
-  __shared__ double lds_s[TABLES ? NSOILCLASS * SC_N : 1];
+  // FP32: default-REAL columns as FP32, the others in FP64 beside them
+  using V = R;
+  constexpr int NV = NVEGCLASS * VC_N, NS = NSOILCLASS * SC_N;
+  __shared__ V lds_v[TABLES ? NV : 1], lds_s[TABLES ? NS : 1];
+  __shared__ V lds_x[TABLES ? NVEGCLASS * VX_N : 1];
+  __shared__ double lds_vd[TABLES && sizeof(V) == 4 ? NVEGCLASS * NVEGD : 1];
+  __shared__ double lds_sd[TABLES && sizeof(V) == 4 ? NS : 1];
   const int64_t mp = a.mp;
   if constexpr (TABLES) {
     // every load issued before the first LDS write: in a loop each waited for
     // its own, one memory latency per 64 (FP64) or 256 values (a day of
     // 262,144 tiles in FP64 16.7 -> 16.4 ms).  Loading them beside the tile's
     // gather, with one wait for both, measured no faster
-    constexpr int B = LateStage<R>::LANES, NV = NVEGCLASS * VC_N, NS = NSOILCLASS * SC_N;
+    constexpr int B = LateStage<R>::LANES;
     double v[(NV + B - 1) / B], s[(NS + B - 1) / B];
 #pragma unroll
     for (int q = 0; q < (NV + B - 1) / B; q++) {
@@ -636,13 +658,23 @@ cbm_kernel(StepArgs a) {
 #pragma unroll
     for (int q = 0; q < (NV + B - 1) / B; q++) {
       const int i = threadIdx.x + q * B;
-      if (i < NV) lds_v[i] = v[q];
+      if (i < NV) lds_v[i] = (V)v[q];
+      if constexpr (sizeof(V) == 4) {
+        const int c = i % VC_N - VC_fes_cor;
+        if (i < NV && c >= 0 && c < NVEGD) lds_vd[i / VC_N * NVEGD + c] = v[q];
+      }
     }
 #pragma unroll
     for (int q = 0; q < (NS + B - 1) / B; q++) {
       const int i = threadIdx.x + q * B;
-      if (i < NS) lds_s[i] = s[q];
+      if (i < NS) lds_s[i] = (V)s[q];
+      if constexpr (sizeof(V) == 4)
+        if (i < NS) lds_sd[i] = s[q];
     }
+    __syncthreads();
+    for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B)
+      lds_x[i] = Stepper<R, FULL, TABLES, MODE, V, true>::derived(
+          i % VX_N, [&](int c) { return (R)lds_v[i / VX_N * VC_N + c]; });
     __syncthreads();
   }
   using Late = LateStage<R>;
@@ -654,7 +686,7 @@ cbm_kernel(StepArgs a) {
   const int64_t t = (int64_t)blockIdx.x * Late::LANES + threadIdx.x;
   const bool live = t < mp;
   TileOut<MODE, CONS> o;
-  if (live) step_tile<R, FULL, TABLES, MODE, CONS, !FULL>(a, t, lds_v, lds_s, o, late);
+  if (live) step_tile<R, FULL, TABLES, MODE, CONS, !FULL, V>(a, t, lds_v, lds_s, o, late, lds_x, lds_vd, lds_sd);
   if constexpr (CONS) {
     // workgroup sums in a fixed order: a butterfly within each wave, then
     // the waves in order

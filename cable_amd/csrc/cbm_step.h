@@ -1,6 +1,6 @@
 // cbm_step.h -- the per-tile CABLE timestep on the GPU (device code).
 //
-// Stepper<R, FULL, TABLES, MODE>::run() performs, for the tile held in `t`,
+// Stepper<R, FULL, TABLES, MODE, V>::run() performs, for the tile held in `t`,
 // one call of the reference's cbm() together with the offline driver's
 // contract around it; see cbm_physics.h for the template parameters and
 // layout.  MODE (StepMode) adds the surrogate's work: MODE_CAPTURE records
@@ -13,11 +13,11 @@
 
 namespace cbm {
 
-template <class R, bool FULL, bool TABLES, int MODE = MODE_PLAIN>
+template <class R, bool FULL, bool TABLES, int MODE = MODE_PLAIN, class V = double, bool DERIVED = false>
 struct Stepper {
   Tile<R> &t;
   const StepArgs &a;
-  const double *vrow, *srow;
+  const ClassRows<V> rows;
   int npass = 0;
   // surrogate: predictions in (MODE_HYBRID), targets out (MODE_CAPTURE), and
   // whether a capped tile's leaf fixed point fell back to the reference's
@@ -51,8 +51,7 @@ struct Stepper {
                      FROZEN_LIMIT = R(0.85), SNMIN = R(1.0);
   static constexpr int LAKES = 16, ICE_VEG = 17, ICE_SOIL = 9;
 
-  CBM_HD Stepper(Tile<R> &t_, const StepArgs &a_, const double *v, const double *s)
-      : t(t_), a(a_), vrow(v), srow(s) {}
+  CBM_HD Stepper(Tile<R> &t_, const StepArgs &a_, const ClassRows<V> &r) : t(t_), a(a_), rows(r) {}
 
   // a / b and x**0.5.  The plain path takes them on the device as the short
   // sequences of cbm_physics.h: the same bits as the compiler's IEEE
@@ -72,6 +71,52 @@ struct Stepper {
     }
 #endif
     return a / b;
+  }
+  // DIV(a, b) with r = recip(b)
+  CBM_HD static R recip(R b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(R) == 8) return refine_reciprocal(b, __builtin_amdgcn_rcp((double)b));
+    else return __builtin_amdgcn_rcpf((float)b);
+#else
+    return K(1.0) / b;
+#endif
+  }
+  CBM_HD static R DIVR(R a, R b, R r) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(R) == 8)
+      return __builtin_amdgcn_div_fixup(corrected_quotient(a, b, r), (double)b, (double)a);
+    else
+      return a * r;
+#else
+    return a / b;
+#endif
+  }
+  // a derived column (ClassRows::x) from its vegetation row
+  template <class P>
+  CBM_HD static R derived(int c, P &&veg) {
+    switch (c) {
+      case VX_rdleaf: return recip(veg(VC_dleaf));
+      case VX_dleaf3: return p3(veg(VC_dleaf));
+      case VX_r2convex: return recip(K(2.0) * veg(VC_convex));
+      case VX_c4ca: return K(4.0) * veg(VC_convex) * veg(VC_alpha);
+      case VX_rd0gs: return recip(veg(VC_d0gs));
+      case VX_ekc: return DIV(veg(VC_ekc), RGAS * TREFK);
+      default: return DIV(veg(VC_eko), RGAS * TREFK);
+    }
+  }
+  CBM_HD R derived(int c) const {
+    if constexpr (DERIVED) {
+      return rows.x[c];
+    } else {
+      return derived(c, [&](int v) {
+        return v == VC_dleaf    ? PV(veg_dleaf, 0)
+               : v == VC_convex ? PV(veg_convex, 0)
+               : v == VC_alpha  ? PV(veg_alpha, 0)
+               : v == VC_d0gs   ? PV(veg_d0gs, 0)
+               : v == VC_ekc    ? PV(veg_ekc, 0)
+                                : PV(veg_eko, 0);
+      });
+    }
   }
   template <class T>
   CBM_HD static T sqrt(T x) {
@@ -438,13 +483,14 @@ struct Stepper {
   }
 
   // src/science/canopy/cbl_dryLeaf.F90:779-877
-  CBM_HD static R ej3x(R parx, R alpha, R convex, R x) {
-    return MAX(K(0.0), K(0.25) * DIV(alpha * parx + x - sqrt(p2(alpha * parx + x) - K(4.0) * convex * alpha * parx * x),
-                                  K(2.0) * convex));
+  // (c4ca = 4 convex alpha, r2 = recip(2 convex))
+  CBM_HD static R ej3x(R parx, R alpha, R convex, R x, R c4ca, R r2) {
+    return MAX(K(0.0), K(0.25) * DIVR(alpha * parx + x - sqrt(p2(alpha * parx + x) - c4ca * parx * x),
+                                   K(2.0) * convex, r2));
   }
-  CBM_HD static R ej4x(R parx, R alpha, R convex, R x) {
-    return MAX(K(0.0), DIV(alpha * parx + x - sqrt(p2(alpha * parx + x) - K(4.0) * convex * alpha * parx * x),
-                           K(2.0) * convex));
+  CBM_HD static R ej4x(R parx, R alpha, R convex, R x, R c4ca, R r2) {
+    return MAX(K(0.0), DIVR(alpha * parx + x - sqrt(p2(alpha * parx + x) - c4ca * parx * x),
+                            K(2.0) * convex, r2));
   }
   CBM_HD static R xvcmxt4(R x) {
     return DIV(exp2(K(0.1) * x - K(2.5)), (K(1.0) + exp(K(0.3) * (K(13.0) - x))) * (K(1.0) + exp(K(0.3) * (x - K(36.0)))));
@@ -660,10 +706,11 @@ struct Stepper {
         R tlfx = c.tlfx;
         R dleaf = PV(veg_dleaf, 0);
         c.ghwet = K(2.0) * sum_gbh;
-        R gras = MAX(K(1.0e-6), K(1.595E8) * fabs(tlfx - tvair) * p3(dleaf));
+        R gras = MAX(K(1.0e-6), K(1.595E8) * fabs(tlfx - tvair) * derived(VX_dleaf3));
         R g25 = root4(gras);
-        c.gbhf[0] = DIV(fvl0 * t.air_cmolar[0] * K(0.5) * DHEAT * (g25), dleaf);
-        c.gbhf[1] = DIV(fvl1 * t.air_cmolar[0] * K(0.5) * DHEAT * (g25), dleaf);
+        const R rdleaf = derived(VX_rdleaf);
+        c.gbhf[0] = DIVR(fvl0 * t.air_cmolar[0] * K(0.5) * DHEAT * (g25), dleaf, rdleaf);
+        c.gbhf[1] = DIVR(fvl1 * t.air_cmolar[0] * K(0.5) * DHEAT * (g25), dleaf, rdleaf);
         c.gbhf[0] = MAX(K(1.e-6), c.gbhf[0]);
         c.gbhf[1] = MAX(K(1.e-6), c.gbhf[1]);
 #pragma unroll
@@ -673,12 +720,13 @@ struct Stepper {
         }
         R frac4 = PV(veg_frac4, 0), vcmax = PV(veg_vcmax, 0);
         R tdiff = tlfx - TREFK;
-        R conkct = PV(veg_conkc0, 0) * exp(DIV(PV(veg_ekc, 0), RGAS * TREFK) * (K(1.0) - DIV(TREFK, tlfx)));
-        R conkot = PV(veg_conko0, 0) * exp(DIV(PV(veg_eko, 0), RGAS * TREFK) * (K(1.0) - DIV(TREFK, tlfx)));
+        R conkct = PV(veg_conkc0, 0) * exp(derived(VX_ekc) * (K(1.0) - DIV(TREFK, tlfx)));
+        R conkot = PV(veg_conko0, 0) * exp(derived(VX_eko) * (K(1.0) - DIV(TREFK, tlfx)));
         tlfxx = tlfx;
         cx1 = conkct * (K(1.0) + DIV(K(0.21), conkot));
         cx2 = K(2.0) * GAM0 * (K(1.0) + GAM1 * tdiff + GAM2 * tdiff * tdiff);
         R alpha = PV(veg_alpha, 0), convex = PV(veg_convex, 0);
+        const R c4ca = derived(VX_c4ca), r2 = derived(VX_r2convex);
         R q0 = t.rad_qcan[0], q1 = t.rad_qcan[1];
         // the C3 and the C4 terms each carry the class's share as a factor:
         // without one they are zero, and their exponentials and roots are
@@ -690,20 +738,20 @@ struct Stepper {
           vcmxt3[1] = t.rad_scalex[1] * temp;
           temp = xejmxt3(tlfx) * PV(veg_ejmax, 0) * (K(1.0) - frac4);
           R ejmxt3_0 = t.rad_scalex[0] * temp, ejmxt3_1 = t.rad_scalex[1] * temp;
-          vx3[0] = ej3x(q0 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_0);
-          vx3[1] = ej3x(q1 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_1);
+          vx3[0] = ej3x(q0 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_0, c4ca, r2);
+          vx3[1] = ej3x(q1 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_1, c4ca, r2);
         }
         if (sizeof(R) == 4 ? c4 : frac4 != K(0.0)) {
           R temp = xvcmxt4(tlfx - TFRZ) * vcmax * frac4;
           vcmxt4[0] = t.rad_scalex[0] * temp;
           vcmxt4[1] = t.rad_scalex[1] * temp;
-          vx4[0] = ej4x(q0 * jtomol * frac4, alpha, convex, vcmxt4[0]);
-          vx4[1] = ej4x(q1 * jtomol * frac4, alpha, convex, vcmxt4[1]);
+          vx4[0] = ej4x(q0 * jtomol * frac4, alpha, convex, vcmxt4[0], c4ca, r2);
+          vx4[1] = ej4x(q1 * jtomol * frac4, alpha, convex, vcmxt4[1], c4ca, r2);
         }
         R cfrd = PV(veg_cfrd, 0);
         rdx[0] = (cfrd * vcmxt3[0] + cfrd * vcmxt4[0]);
         rdx[1] = (cfrd * vcmxt3[1] + cfrd * vcmxt4[1]);
-        R a1 = DIV(PV(veg_a1gs, 0), K(1.0) + DIV(c.dsx, PV(veg_d0gs, 0)));
+        R a1 = DIV(PV(veg_a1gs, 0), K(1.0) + DIVR(c.dsx, PV(veg_d0gs, 0), derived(VX_rd0gs)));
         gs_coeff[0] = DIV(fwsoil, c.csx[0] - K(0.0)) * a1;
         gs_coeff[1] = DIV(fwsoil, c.csx[1] - K(0.0)) * a1;
         // one leaf's assimilation, leaf-surface CO2 and conductances; `has`:
