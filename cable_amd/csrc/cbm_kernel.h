@@ -300,10 +300,17 @@ constexpr int field_phase(int id) {
 // host arrays, under the sanitizers.
 // xtab: the derived columns (STAGE); vdtab/sdtab: FP64 columns beside an FP32
 // table (ClassRows).
-template <class R, bool FULL, bool TABLES, int MODE, bool CONS, bool STAGE = false, class V = double>
+// tables(): called by every lane once the gather is under way, stages the tables;
+// `live`: the lane's tile is its own (else it gathers another's and ends there).
+struct NoTables {
+  CBM_HD void operator()() const {}
+};
+template <class R, bool FULL, bool TABLES, int MODE, bool CONS, bool STAGE = false, class V = double,
+          class Tables = NoTables>
 CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> *vtab,
                       const std::common_type_t<V> *stab, TileOut<MODE, CONS> &o, LateStage<R> late_lds = {},
-                      const V *xtab = nullptr, const double *vdtab = nullptr, const double *sdtab = nullptr) {
+                      const V *xtab = nullptr, const double *vdtab = nullptr, const double *sdtab = nullptr,
+                      Tables &&tables = Tables(), bool live = true) {
   const int64_t mp = a.mp;
   FieldTable F = (FieldTable)(uintptr_t)a.F;
   Tile<R> T;
@@ -398,6 +405,8 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
 #undef LDS_
 #undef LDD_
   }
+  tables();
+  if (!live) return;
   const int iv = T.veg_iveg[0] - 1, is = T.soil_isoilm[0] - 1;
   ClassRows<V> rows;
   if constexpr (TABLES) {
@@ -638,45 +647,52 @@ cbm_kernel(StepArgs a) {
   __shared__ double lds_vd[TABLES && sizeof(V) == 4 ? NVEGCLASS * NVEGD : 1];
   __shared__ double lds_sd[TABLES && sizeof(V) == 4 ? NS : 1];
   const int64_t mp = a.mp;
+  constexpr int B = LateStage<R>::LANES;
+  double tv[TABLES ? (NV + B - 1) / B : 1], ts[TABLES ? (NS + B - 1) / B : 1];
   if constexpr (TABLES) {
     // every load issued before the first LDS write: in a loop each waited for
     // its own, one memory latency per 64 (FP64) or 256 values (a day of
-    // 262,144 tiles in FP64 16.7 -> 16.4 ms).  Loading them beside the tile's
-    // gather, with one wait for both, measured no faster
-    constexpr int B = LateStage<R>::LANES;
-    double v[(NV + B - 1) / B], s[(NS + B - 1) / B];
+    // 262,144 tiles in FP64 16.7 -> 16.4 ms)
 #pragma unroll
     for (int q = 0; q < (NV + B - 1) / B; q++) {
       const int i = threadIdx.x + q * B;
-      v[q] = a.vtab[i < NV ? i : 0];
+      tv[q] = a.vtab[i < NV ? i : 0];
     }
 #pragma unroll
     for (int q = 0; q < (NS + B - 1) / B; q++) {
       const int i = threadIdx.x + q * B;
-      s[q] = a.stab[i < NS ? i : 0];
+      ts[q] = a.stab[i < NS ? i : 0];
     }
-#pragma unroll
-    for (int q = 0; q < (NV + B - 1) / B; q++) {
-      const int i = threadIdx.x + q * B;
-      if (i < NV) lds_v[i] = (V)v[q];
-      if constexpr (sizeof(V) == 4) {
-        const int c = i % VC_N - VC_fes_cor;
-        if (i < NV && c >= 0 && c < NVEGD) lds_vd[i / VC_N * NVEGD + c] = v[q];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < (NS + B - 1) / B; q++) {
-      const int i = threadIdx.x + q * B;
-      if (i < NS) lds_s[i] = (V)s[q];
-      if constexpr (sizeof(V) == 4)
-        if (i < NS) lds_sd[i] = s[q];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B)
-      lds_x[i] = Stepper<R, FULL, TABLES, MODE, V, true>::derived(
-          i % VX_N, [&](int c) { return (R)lds_v[i / VX_N * VC_N + c]; });
-    __syncthreads();
   }
+  // the tables to LDS, once the tile's gather is under way too, so that the
+  // wave waits for memory once (barriers that wait for LDS only): a day of
+  // 262,144 tiles in FP64 15.7 -> 15.4 ms, of 1,048,576 in mixed precision 18.1
+  // -> 18.0 ms
+  auto tables = [&]() {
+    if constexpr (TABLES) {
+#pragma unroll
+      for (int q = 0; q < (NV + B - 1) / B; q++) {
+        const int i = threadIdx.x + q * B;
+        if (i < NV) lds_v[i] = (V)tv[q];
+        if constexpr (sizeof(V) == 4) {
+          const int c = i % VC_N - VC_fes_cor;
+          if (i < NV && c >= 0 && c < NVEGD) lds_vd[i / VC_N * NVEGD + c] = tv[q];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < (NS + B - 1) / B; q++) {
+        const int i = threadIdx.x + q * B;
+        if (i < NS) lds_s[i] = (V)ts[q];
+        if constexpr (sizeof(V) == 4)
+          if (i < NS) lds_sd[i] = ts[q];
+      }
+      lds_barrier();
+      for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B)
+        lds_x[i] = Stepper<R, FULL, TABLES, MODE, V, true>::derived(
+            i % VX_N, [&](int c) { return (R)lds_v[i / VX_N * VC_N + c]; });
+      lds_barrier();
+    }
+  };
   using Late = LateStage<R>;
   __shared__ typename DevT<R, 'F'>::type late_f[FULL ? 1 : Late::NF * Late::LANES];
   __shared__ double late_d[FULL ? 1 : Late::ND * Late::LANES];
@@ -686,7 +702,12 @@ cbm_kernel(StepArgs a) {
   const int64_t t = (int64_t)blockIdx.x * Late::LANES + threadIdx.x;
   const bool live = t < mp;
   TileOut<MODE, CONS> o;
-  if (live) step_tile<R, FULL, TABLES, MODE, CONS, !FULL, V>(a, t, lds_v, lds_s, o, late, lds_x, lds_vd, lds_sd);
+  if constexpr (FULL) {
+    if (live) step_tile<R, FULL, TABLES, MODE, CONS, false, V>(a, t, lds_v, lds_s, o);
+  } else {
+    step_tile<R, FULL, TABLES, MODE, CONS, true, V>(a, live ? t : mp - 1, lds_v, lds_s, o, late, lds_x, lds_vd,
+                                                    lds_sd, tables, live);
+  }
   if constexpr (CONS) {
     // workgroup sums in a fixed order: a butterfly within each wave, then
     // the waves in order
