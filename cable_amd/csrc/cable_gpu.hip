@@ -185,6 +185,10 @@ struct cable_gpu_ctx {
   unsigned char *h_stage = nullptr, *d_stage = nullptr;
   size_t stage_bytes = 0;
   std::vector<hipEvent_t> xev;      // a download's copies, one each
+  // ---- a run's step arguments ----
+  std::vector<StepArgs> h_steps;
+  StepArgs *d_steps = nullptr;
+  int steps_cap = 0;
 };
 
 namespace {
@@ -517,6 +521,38 @@ StepArgs make_args(const cable_gpu_ctx *c, void **tab, int ktau, double dels, in
   return a;
 }
 
+// The plain resident steps of one launch, at most: with 48 a launch of 4,194,304
+// tiles lasts 0.1 s.
+constexpr int RUN_STEPS = 48;
+
+// the arguments of resident steps k0 .. k0 + nsteps - 1 to c->d_steps
+int set_steps(cable_gpu_ctx *c, int k0, int nsteps, double dels) {
+  std::vector<StepArgs> &h = c->h_steps;
+  h.clear();
+  for (int k = k0; k < k0 + nsteps; k++) {
+    h.push_back(make_args(c, c->d_tab_run, k + 1, dels, (int64_t)(k - c->forc_k0) * c->mp));
+    if (k > k0) h.back().first_call = 0;
+  }
+  if (nsteps > c->steps_cap) {
+    if (c->d_steps) HIPCHECK(hipFree(c->d_steps));
+    c->d_steps = nullptr;
+    c->steps_cap = 0;
+    HIPCHECK(hipMalloc((void **)&c->d_steps, sizeof(StepArgs) * (size_t)nsteps));
+    c->steps_cap = nsteps;
+  }
+  HIPCHECK(hipMemcpyAsync(c->d_steps, h.data(), sizeof(StepArgs) * h.size(), hipMemcpyHostToDevice, c->stream));
+  return CABLE_OK;
+}
+
+// n plain resident steps, the first the q-th of set_steps
+hipError_t launch_run(const cable_gpu_ctx *c, int q, int n) {
+  StepArgs a = c->h_steps[(size_t)q];
+  a.nsteps = n;
+  a.steps = c->d_steps + q;
+  return c->precision == CABLE_PREC_MIXED ? launch_run_mixed(a, c->mp, c->stream)
+                                          : launch_run_fp64(a, c->mp, c->stream);
+}
+
 hipError_t launch(const cable_gpu_ctx *c, const StepArgs &a, bool full) {
   return c->precision == CABLE_PREC_MIXED ? launch_mixed(full, a, c->mp, c->stream)
                                           : launch_fp64(full, a, c->mp, c->stream);
@@ -644,7 +680,7 @@ int cable_gpu_destroy(cable_gpu_ctx *c) {
   if (c->d_stab) hipFree(c->d_stab);
   if (c->d_npass) hipFree(c->d_npass);
   void *sur[] = {c->cons_part, c->cons_acc, c->hyb, c->sx, c->sy, c->scount, c->sparams, c->snorm, c->pred, c->swt,
-                 c->nfallback, c->d_lit, c->d_litblk, c->d_order};
+                 c->nfallback, c->d_lit, c->d_litblk, c->d_order, c->d_steps};
   for (void *p : sur)
     if (p) hipFree(p);
   if (c->h_stage) hipHostFree(c->h_stage);
@@ -1476,11 +1512,19 @@ int cable_gpu_run(cable_gpu_ctx *c, int k0, int nsteps, double dels) {
   HIPCHECK(hipMemsetAsync(c->d_npass, 0, sizeof(unsigned long long), c->stream));
   c->hyb_valid = false;   // the plain step does not keep the surrogate's inputs
   HIPCHECK(hipEventRecord(c->ev0, c->stream));
-  for (int k = k0; k < k0 + nsteps; k++) {
-    StepArgs a = make_args(c, c->d_tab_run, k + 1, dels, (int64_t)(k - c->forc_k0) * c->mp);
-    if (c->cons_on) a.cons_part = c->cons_part;
-    hipError_t e = launch(c, a, false);
-    if (e == hipSuccess && c->cons_on) e = launch_cons_reduce(c);
+  if (const int r = set_steps(c, k0, nsteps, dels)) return r;
+  for (int k = k0, n; k < k0 + nsteps; k += n) {
+    hipError_t e;
+    if (c->cons_on) {
+      n = 1;
+      StepArgs a = c->h_steps[(size_t)(k - k0)];
+      a.cons_part = c->cons_part;
+      e = launch(c, a, false);
+      if (e == hipSuccess) e = launch_cons_reduce(c);
+    } else {
+      n = std::min(RUN_STEPS, k0 + nsteps - k);
+      e = launch_run(c, k - k0, n);
+    }
     if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_run launch: %s", hipGetErrorString(e));
     c->first_call = false;
   }
@@ -1624,9 +1668,12 @@ int cable_gpu_run_hybrid(cable_gpu_ctx *c, int k0, int nsteps, double dels, int 
   HIPCHECK(hipMemsetAsync(c->nfallback, 0, sizeof(unsigned long long), c->stream));
   HIPCHECK(hipMemsetAsync(c->d_npass, 0, sizeof(unsigned long long), c->stream));
   HIPCHECK(hipEventRecord(c->ev0, c->stream));
+  if ((r = set_steps(c, k0, nsteps, dels))) return r;
+  std::vector<int> timed;  // the first step of each launch
   unsigned long long lit = 0;
-  for (int k = k0; k < k0 + nsteps; k++) {
-    StepArgs a = make_args(c, c->d_tab_run, k + 1, dels, (int64_t)(k - c->forc_k0) * c->mp);
+  for (int k = k0, n; k < k0 + nsteps; k += n) {
+    n = 1;
+    StepArgs a = c->h_steps[(size_t)(k - k0)];
     if ((k - k0) % LIT_CHUNK == 0) {
       // the steps of the next chunk with a leaf-bearing tile in daylight (one
       // scan of their shortwave and one wait per 64 steps)
@@ -1649,6 +1696,10 @@ int cable_gpu_run_hybrid(cable_gpu_ctx *c, int k0, int nsteps, double dels, int 
     const bool day = (lit >> s) & 1ull;
     const bool next_day = s + 1 == LIT_CHUNK || k + 1 == k0 + nsteps || ((lit >> (s + 1)) & 1ull);
     const int mode = day ? MODE_HYBRID : next_day ? MODE_UNLIT : MODE_PLAIN;
+    // plain steps in a row: one launch
+    while (mode == MODE_PLAIN && n < RUN_STEPS && s + n + 1 < LIT_CHUNK && k + n + 1 < k0 + nsteps &&
+           !((lit >> (s + n)) & 3ull))
+      n++;
     a.hyb = c->hyb;
     a.hyb_valid = c->hyb_valid ? 1 : 0;
     a.norm = c->snorm;
@@ -1666,8 +1717,10 @@ int cable_gpu_run_hybrid(cable_gpu_ctx *c, int k0, int nsteps, double dels, int 
     // the capped step; a tile the residual test rejects falls back to the
     // reference's iteration within the same launch
     if (c->launch_timing) HIPCHECK(hipEventRecord(ev[2], c->stream));
-    if (e == hipSuccess) e = launch_mixed_mode(mode, a, c->mp, c->stream);
+    if (e == hipSuccess)
+      e = mode == MODE_PLAIN ? launch_run(c, k - k0, n) : launch_mixed_mode(mode, a, c->mp, c->stream);
     if (c->launch_timing) HIPCHECK(hipEventRecord(ev[3], c->stream));
+    timed.push_back(k - k0);
     if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_run_hybrid launch: %s", hipGetErrorString(e));
     c->first_call = false;
     c->hyb_valid = true;
@@ -1682,7 +1735,8 @@ int cable_gpu_run_hybrid(cable_gpu_ctx *c, int k0, int nsteps, double dels, int 
   HIPCHECK(hipMemcpy(&fb, c->nfallback, sizeof fb, hipMemcpyDeviceToHost));
   c->last_infer_ms = c->last_step_ms = 0.0;
   if (!c->launch_timing) c->last_step_ms = ms;
-  for (int k = 0; c->launch_timing && k < nsteps; k++) {
+  for (size_t q = 0; c->launch_timing && q < timed.size(); q++) {
+    const int k = timed[q];
     float a = 0.f, b = 0.f;
     HIPCHECK(hipEventElapsedTime(&a, c->kev[4 * (size_t)k], c->kev[4 * (size_t)k + 1]));
     HIPCHECK(hipEventElapsedTime(&b, c->kev[4 * (size_t)k + 2], c->kev[4 * (size_t)k + 3]));

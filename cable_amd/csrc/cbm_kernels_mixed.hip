@@ -8,9 +8,8 @@
 namespace cbm {
 
 hipError_t launch_mixed(bool full, const StepArgs &a, int64_t mp, hipStream_t stream) {
-  if (full) return launch_cbm<float, true, false>(a, mp, stream);
-  return a.cons_part ? launch_cbm<float, false, true, MODE_PLAIN, true>(a, mp, stream)
-                     : launch_cbm<float, false, true>(a, mp, stream);
+  return full ? launch_cbm<float, true, false>(a, mp, stream)
+              : launch_cbm<float, false, true, MODE_PLAIN, true>(a, mp, stream);
 }
 
 hipError_t launch_mixed_mode(int mode, const StepArgs &a, int64_t mp, hipStream_t stream) {
@@ -18,7 +17,7 @@ hipError_t launch_mixed_mode(int mode, const StepArgs &a, int64_t mp, hipStream_
     case MODE_CAPTURE: return launch_cbm<float, false, true, MODE_CAPTURE>(a, mp, stream);
     case MODE_HYBRID: return launch_cbm<float, false, true, MODE_HYBRID>(a, mp, stream);
     case MODE_UNLIT: return launch_cbm<float, false, true, MODE_UNLIT>(a, mp, stream);
-    default: return launch_cbm<float, false, true, MODE_PLAIN>(a, mp, stream);
+    default: return hipErrorInvalidValue;
   }
 }
 

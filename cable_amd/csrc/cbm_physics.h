@@ -131,6 +131,8 @@ struct StepArgs {
   int64_t mp;
   int64_t foff;          // element offset of this step in the forcing arrays
   int ktau;
+  int nsteps;            // resident plain step: the steps of a launch, and the
+  const StepArgs *steps;  // arguments of each, in device memory
   int first_call;        // first soil_snow call of the run (gammzz(:,1) init)
   int driver;            // 1: the offline driver's step (its contract around
                          // cbm and the balance checks); 0: cbm alone
