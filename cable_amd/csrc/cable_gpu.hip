@@ -417,6 +417,7 @@ hipError_t stage_down(cable_gpu_ctx *c, size_t bytes, bool copy, F &&drain) {
     }
     drain(q * XFER_PIECE, std::min(bytes, (q + 1) * XFER_PIECE));
   });
+  if (err != hipSuccess) (void)hipStreamSynchronize(c->stream);  // the buffer is not left in use
   return (hipError_t)err.load();
 }
 

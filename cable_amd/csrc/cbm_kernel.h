@@ -351,7 +351,7 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
     LDD_(ssnow_wb, 1) LDD_(ssnow_wbice, 1)
     // the canopy reads only the top soil and snow layer; the deeper layers,
     // snow layers, carbon pools, gammzz(:,1) and the balance accumulators
-    // are loaded after the canopy (Stepper::run's `late`).  Soil liquid
+    // are taken after the canopy (Stepper::run's `late`).  Soil liquid
     // water as the previous step left it (wb - wbice), before this step's
     // lake fix-up:
 #pragma unroll

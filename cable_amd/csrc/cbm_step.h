@@ -2141,11 +2141,11 @@ struct Stepper {
     run([] {}, [] {}, [] {}, [] {});
   }
   // `late` runs after the canopy and before soil and snow: the resident
-  // kernel loads there the state that only soil, snow, carbon and the
-  // balances read, so it is not held in registers through the canopy
-  // iteration.  `tail` runs after soil and snow, before the flux totals and
-  // carbon: the resident kernel issues there the loads of the driver's
-  // running sums, which sumcflux reads after the step.
+  // kernel takes there, from LDS, the state that only soil, snow, carbon and
+  // the balances read, so it is not held in registers through the canopy
+  // iteration (the drop-in kernel loads it there).  `tail` runs after soil and
+  // snow, before the flux totals and carbon: the resident kernel takes there
+  // the driver's running sums, which sumcflux reads after the step.
   // `stash` runs before the canopy, `settled` in it before the leaf iteration,
   // when the radiation, roughness and air diagnostics have their last values.
   template <class Late, class Tail, class Stash, class Settled>
