@@ -530,7 +530,7 @@ struct Stepper {
       const R d = (b ? -s : s) - coef1z;
       return DIV(b ? K(2.0) * coef0z : d, b ? d : K(2.0) * coef2z);
     }
-    const bool linear = fabs(coef2z) < K(1.0e-9);
+    const bool linear = !(fabs(coef2z) >= K(1.0e-9));
     return DIV(linear ? -coef0z : -coef1z + s, linear ? coef1z : K(2.0) * coef2z);
   }
 
@@ -563,25 +563,28 @@ struct Stepper {
     R z[3];
 #pragma unroll
     for (int q = 0; q < 3; q++) z[q] = larger_root(coef2[q], coef1[q], coef0[q]);
-    bool none[3];
+    // a limit whose coefficients give neither form keeps the reference's initial
+    // value: both too small, or (FP64) NaN (in coef1, whose terms hold the
+    // factors of coef2, so that two compares a limit tell)
+    bool solved[3];
 #pragma unroll
     for (int q = 0; q < 3; q++)
-      none[q] = sizeof(R) == 8 && fabs(coef2[q]) < K(1.0e-9) && fabs(coef1[q]) < K(1.0e-9);
+      solved[q] = sizeof(R) == 4 || fabs(coef2[q]) >= K(1.0e-9) || fabs(coef1[q]) >= K(1.0e-9);
     if (sizeof(R) == 4 && (fabs(coef2[0]) < K(1.0e-9) || fabs(coef2[1]) < K(1.0e-9) || fabs(coef2[2]) < K(1.0e-9))) {
 #pragma unroll
       for (int q = 0; q < 3; q++)
         if (fabs(coef2[q]) < K(1.0e-9)) {
           z[q] = DIV(-coef0[q], coef1[q]);
-          none[q] = fabs(coef1[q]) < K(1.0e-9);
+          solved[q] = fabs(coef1[q]) >= K(1.0e-9);
         }
     }
     R ciz = MAX(K(0.0), z[0]);
     R anrubiscoz = DIV(vcmxt3z * (ciz - cx2z / K(2.0)), ciz + cx1z) + vcmxt4z - rdxz;
-    anrubiscoz = none[0] ? K(0.0) : anrubiscoz;
+    anrubiscoz = solved[0] ? anrubiscoz : K(0.0);
     ciz = MAX(K(0.0), z[1]);
     R anrubpz = DIV(vx3z * (ciz - cx2z / K(2.0)), ciz + cx2z) + vx4z - rdxz;
-    anrubpz = none[1] ? K(99999.0) : anrubpz;
-    const R ansinkz = none[2] ? K(99999.0) : z[2];
+    anrubpz = solved[1] ? anrubpz : K(99999.0);
+    const R ansinkz = solved[2] ? z[2] : fabs(coef1[2]) < K(1.0e-9) ? K(99999.0) : K(0.0);
     return MIN(MIN(anrubiscoz, anrubpz), ansinkz);
   }
 
