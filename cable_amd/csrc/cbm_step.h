@@ -674,7 +674,16 @@ struct Stepper {
     const R tvair = t.met_tvair[0], tk = t.met_tk[0];
     const R fvl0 = t.rad_fvlai[0], fvl1 = t.rad_fvlai[1];
     const bool leaves = fvl0 + fvl1 > LAI_THRESH;
-    const bool c4 = PV(veg_frac4, 0) != K(0.0);
+    // whether the class has C3 and C4 leaves; in FP64 also set where the terms
+    // of the absent ones are not zero: a share of zero times NaN or infinity
+    bool c3 = true, c4 = PV(veg_frac4, 0) != K(0.0);
+    if constexpr (sizeof(R) == 8) {
+      const R convex = fabs(PV(veg_convex, 0));
+      const bool odd = !(fabs(PV(veg_vcmax, 0)) < K(1e30) && fabs(PV(veg_ejmax, 0)) < K(1e30) &&
+                         fabs(PV(veg_alpha, 0)) < K(1e30) && convex > K(0.0) && convex < K(1e30));
+      c3 = PV(veg_frac4, 0) != K(1.0) || odd;
+      c4 = c4 || odd;
+    }
     // the reference's fixed count of 20 passes.  The hybrid polishes the
     // start of a sunlit leaf-bearing tile with a.max_passes passes and then
     // checks it by its leaf energy-balance residual: the leaf
@@ -739,8 +748,15 @@ struct Stepper {
         // the C3 and the C4 terms each carry the class's share as a factor:
         // without one they are zero, and their exponentials and roots are
         // left out (in FP32 the C4 terms only: the branch around the C3 terms
-        // waits for the class table and costs more than it saves)
-        if (sizeof(R) == 4 || frac4 != K(1.0)) {
+        // waits for the class table and costs more than it saves).  A leaf
+        // iterate near or below 0 K, where the exponentials overflow, keeps
+        // them, and with them the reference's NaN
+        if constexpr (sizeof(R) == 8) {
+          const bool hot = !(tlfx >= K(64.0) && tlfx < K(1024.0));
+          c3 = c3 || hot;
+          c4 = c4 || hot;
+        }
+        if (sizeof(R) == 4 || c3) {
           R temp = xvcmxt3(tlfx) * vcmax * (K(1.0) - frac4);
           vcmxt3[0] = t.rad_scalex[0] * temp;
           vcmxt3[1] = t.rad_scalex[1] * temp;
@@ -749,7 +765,7 @@ struct Stepper {
           vx3[0] = ej3x(q0 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_0, c4ca, r2);
           vx3[1] = ej3x(q1 * jtomol * (K(1.0) - frac4), alpha, convex, ejmxt3_1, c4ca, r2);
         }
-        if (sizeof(R) == 4 ? c4 : frac4 != K(0.0)) {
+        if (c4) {
           R temp = xvcmxt4(tlfx - TFRZ) * vcmax * frac4;
           vcmxt4[0] = t.rad_scalex[0] * temp;
           vcmxt4[1] = t.rad_scalex[1] * temp;

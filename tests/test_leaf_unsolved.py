@@ -25,6 +25,13 @@ FORMS = {
     "no_curvature": ("veg%convex", 0.0),
     "infinite_slope": ("veg%a1gs", np.inf),
 }
+# on the CPU only, where the step has the oracle's elementary functions: a leaf
+# iterate below 0 K amplifies their last place
+CPU_FORMS = {
+    **FORMS,
+    "no_electron_transport_limit": ("veg%ejmax", np.inf),
+    "air_below_0K": ("met%tk", -1.0),
+}
 
 
 def _case(field, value, with_sens):
@@ -61,7 +68,7 @@ def _differences(got, want, sens):
     return bad
 
 
-@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("form", CPU_FORMS)
 def test_host_build_matches_oracle_without_a_root(tmp_path_factory, tmp_path, form):
     if not (os.path.exists(HIPCC) and os.path.exists(CLANG)):
         pytest.skip("hipcc not found")
@@ -70,7 +77,7 @@ def test_host_build_matches_oracle_without_a_root(tmp_path_factory, tmp_path, fo
     if not os.path.exists(exe):
         subprocess.run([HIPCC] + BASE + ["-c", SRC, "-o", exe + ".o"], check=True, capture_output=True)
         subprocess.run([CLANG, exe + ".o", "-o", exe], check=True, capture_output=True)
-    wl, pre, post, sens = _case(*FORMS[form], False)
+    wl, pre, post, sens = _case(*CPU_FORMS[form], False)
     got, _ = _run(exe, tmp_path, wl, 1, True, 0, [pre])
     assert not _differences(got[0], post, sens)
 
