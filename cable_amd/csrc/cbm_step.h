@@ -1109,14 +1109,17 @@ struct Stepper {
       const R zr = iter == 1 ? ZETA0 : iter == 2 ? zeta1 : iter == 3 ? zeta2 : zeta3;
       // the four profile functions take the sign of zr (the heights are
       // positive): one branch, so that their chains of roots, logarithms and
-      // exponentials overlap; at zero, in the first pass, they are constants.
+      // exponentials overlap; at zero, in the first pass, they are constants
+      // (NaN for an infinite height, as zero times it is).
       // A day of 262,144 tiles in FP64 15.4 -> 15.1 ms, of 4,093 tiles 5.21 ->
       // 5.13 ms, of 1,048,576 in mixed precision 18.1 -> 18.0 ms.
       R mz = MAX(zruffs - disp, z0soilsn);
       R psim_1, psim_2, psis_1, psis_2;
       if (iter == 1) {
-        psim_1 = psim_2 = psim_stable(ZETA0);
-        psis_1 = psis_2 = psis_stable(ZETA0);
+        psim_1 = psim_stable(ZETA0) + ZETA0 * zuv;
+        psim_2 = psim_stable(ZETA0) + ZETA0 * z0m;
+        psis_1 = psis_stable(ZETA0);
+        psis_2 = psis_stable(ZETA0) + ZETA0 * mz;
       } else if (stable(zr)) {
         psim_1 = psim_stable(DIV(zr * zuv, ztq));
         psim_2 = psim_stable(DIV(zr * z0m, ztq));

@@ -26,11 +26,12 @@ FORMS = {
     "infinite_slope": ("veg%a1gs", np.inf),
 }
 # on the CPU only, where the step has the oracle's elementary functions: a leaf
-# iterate below 0 K amplifies their last place
+# iterate below 0 K and an infinite height amplify their last place
 CPU_FORMS = {
     **FORMS,
     "no_electron_transport_limit": ("veg%ejmax", np.inf),
     "air_below_0K": ("met%tk", -1.0),
+    "infinite_height": ("rough%za_uv", np.inf),
 }
 
 
