@@ -3,6 +3,7 @@ source tree):
 
 * cable_amd/libcable_gpu.so  -- HIP kernels and C ABI (include/cable_gpu.h),
   compiled for gfx950 with hipcc;
+* tests/libgpu_quotient.so -- a test's kernel (tests/gpu_quotient.hip);
 * oracle/liboracle.so, oracle/_ref/*  -- the test oracle and, when the
   reference tree is present, the compiled reference (oracle/Makefile).
 """
@@ -24,7 +25,8 @@ HIPCC_FLAGS = [
     "-Wno-unused-result",
 ]
 # per translation unit: the plain FP64 path reproduces the reference's
-# rounding (no FMA contraction, IEEE division and square root); the mixed
+# rounding (no FMA contraction; the step's quotients and roots are
+# cbm_physics.h's, IEEE's bits by shorter sequences); the mixed
 # path is held to its flux tolerance and may contract within an expression
 # and use the hardware approximations of the elementary functions
 TU_FLAGS = {
@@ -96,6 +98,21 @@ def build_gpu(verbose=False):
     return LIB
 
 
+def build_test_kernels(verbose=False):
+    """tests/libgpu_quotient.so: the FP64 step's quotients and roots on host
+    operands, with the flags of the FP64 kernels."""
+    out = os.path.join(ROOT, "tests", "libgpu_quotient.so")
+    r = subprocess.run([hipcc()] + HIPCC_FLAGS + TU_FLAGS["cbm_run_fp64.hip"] +
+                       ["-shared", "-o", out + ".tmp", os.path.join(ROOT, "tests", "gpu_quotient.hip")],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stderr)
+        raise RuntimeError("hipcc failed for tests/gpu_quotient.hip")
+    os.replace(out + ".tmp", out)
+    if verbose:
+        print("built", out)
+
+
 def build_oracle(with_reference=True, verbose=False):
     targets = ["oracle"]
     if with_reference and os.path.isdir("/root/reference/src"):
@@ -113,6 +130,7 @@ def build_oracle(with_reference=True, verbose=False):
 
 def build_all(verbose=True):
     build_gpu(verbose)
+    build_test_kernels(verbose)
     build_oracle(verbose=verbose)
 
 
