@@ -224,11 +224,33 @@ struct TileOut {
 // 256-lane workgroup's LDS in FP32, 31 KB of a wave's in FP64: with the
 // tables, two and four workgroups per CU fit the 160 KB.  A lane's values are
 // LANES apart.
+//
+// The fields, X(id, k0, k1): values k0 .. k1-1 of a field.  One list each drives
+// the gather, the write to LDS and the read after the canopy.
+#define LATE_REAL(X) \
+  X(ssnow_tgg, 1, 6) X(ssnow_tggsn, 1, 3) X(ssnow_smass, 0, 3) X(ssnow_ssdn, 0, 3) X(bgc_cplant, 0, 3) X(bgc_csoil, 0, 2)
+#define LATE_FP64(X) \
+  X(ssnow_wb, 1, 6) X(ssnow_wbice, 1, 6) X(drv_owb, 0, 1) X(bal_ebal_tot, 0, 1) X(bal_wbal_tot, 0, 1) \
+  X(bal_precip_tot, 0, 1) X(bal_rnoff_tot, 0, 1) X(bal_evap_tot, 0, 1) X(bal_radbalsum, 0, 1) X(ssnow_gammzz, 0, 1)
+#define LATE_SUMS(X) \
+  X(sum_flux_sumpn, 0, 1) X(sum_flux_sumrp, 0, 1) X(sum_flux_sumrpw, 0, 1) X(sum_flux_sumrpr, 0, 1) \
+  X(sum_flux_sumrs, 0, 1) X(sum_flux_sumrd, 0, 1) X(sum_flux_dsumpn, 0, 1) X(sum_flux_dsumrp, 0, 1) \
+  X(sum_flux_dsumrd, 0, 1)
+// parked: in both precisions, and in FP64 only
+#define PARKED(X) \
+  X(ssnow_wbtot1, 0, 1) X(ssnow_wbtot2, 0, 1) X(ssnow_wb_lake, 0, 1) X(ssnow_snage, 0, 1) X(ssnow_ssdnn, 0, 1) \
+  X(rad_albedo, 0, 2) X(veg_vlai, 0, 1)
+#define PARKED_FP64(X) \
+  X(met_fsd, 0, 2) X(met_precip, 0, 1) X(met_precip_sn, 0, 1) X(ssnow_otss, 0, 1) X(rad_qcan, 2, 4) X(rad_flws, 0, 1)
 template <class R>
 struct LateStage {
   static constexpr int LANES = sizeof(R) == 8 ? 64 : 256;  // the kernel's workgroup
+#define COUNT_(id, k0, k1) +(k1 - k0)
   // default REAL values (the carbon sums from SUM0, the parked values from PARK0), FP64 values
-  static constexpr int SUM0 = 18, PARK0 = SUM0 + 9, NF = PARK0 + (sizeof(R) == 8 ? 16 : 8), ND = 18;
+  static constexpr int SUM0 = 0 LATE_REAL(COUNT_), PARK0 = SUM0 LATE_SUMS(COUNT_),
+                       NF = PARK0 PARKED(COUNT_) + (sizeof(R) == 8 ? 0 PARKED_FP64(COUNT_) : 0),
+                       ND = 0 LATE_FP64(COUNT_);
+#undef COUNT_
   typename DevT<R, 'F'>::type *f = nullptr;
   double *d = nullptr;
 };
@@ -298,8 +320,9 @@ constexpr int field_phase(int id) {
 // the results.  vtab/stab are the class tables (TABLES), staged in LDS by the
 // kernel.  Host and device code: the test suite also runs it on the CPU, on
 // host arrays, under the sanitizers.
-// xtab: the derived columns (STAGE); vdtab/sdtab: FP64 columns beside an FP32
-// table (ClassRows).
+// STAGE: the caller gives the lane's LateStage slots, LANES apart, and xtab, the
+// derived columns (else, on the host, the slots are the step's own).
+// vdtab/sdtab: FP64 columns beside an FP32 table (ClassRows).
 // tables(): called by every lane once the gather is under way, stages the tables;
 // `live`: the lane's tile is its own (else it gathers another's and ends there).
 struct NoTables {
@@ -314,9 +337,18 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
   const int64_t mp = a.mp;
   FieldTable F = (FieldTable)(uintptr_t)a.F;
   Tile<R> T;
-  // (STAGE) the late state on its way to LDS
-  typename DevT<R, 'F'>::type lf[LateStage<R>::PARK0];
-  double ld_[LateStage<R>::ND];
+  // (resident) the late state on its way to its slots
+  using Late = LateStage<R>;
+  typename DevT<R, 'F'>::type lf[Late::PARK0];
+  double ld_[Late::ND];
+  constexpr bool OWN = !FULL && !STAGE;
+  constexpr int L = STAGE ? Late::LANES : 1;
+  typename DevT<R, 'F'>::type own_f[OWN ? Late::NF : 1];
+  double own_d[OWN ? Late::ND : 1];
+  if constexpr (OWN) {
+    late_lds.f = own_f;
+    late_lds.d = own_d;
+  }
   // ---- gather ----
   if constexpr (FULL) {
 #define PARAM ROLE_PARAM
@@ -384,21 +416,14 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
       T.met_ca[0] = (R)a.ca;
       T.met_doy[0] = (R)a.doy;
     }
-    if constexpr (STAGE) {
+    {
       using DT = typename DevT<R, 'F'>::type;
       int n = 0, m = 0;
 #define LF_(id, k0, k1) \
   { _Pragma("unroll") for (int k = k0; k < k1; k++) lf[n++] = ld<DT>(F[CABLE_F_##id], (int64_t)k * mp, t); }
 #define LD_(id, k0, k1) \
   { _Pragma("unroll") for (int k = k0; k < k1; k++) ld_[m++] = ld<double>(F[CABLE_F_##id], (int64_t)k * mp, t); }
-      LF_(ssnow_tgg, 1, 6) LF_(ssnow_tggsn, 1, 3) LF_(ssnow_smass, 0, 3) LF_(ssnow_ssdn, 0, 3) LF_(bgc_cplant, 0, 3)
-      LF_(bgc_csoil, 0, 2)
-      LD_(ssnow_wb, 1, 6) LD_(ssnow_wbice, 1, 6) LD_(drv_owb, 0, 1) LD_(bal_ebal_tot, 0, 1) LD_(bal_wbal_tot, 0, 1)
-      LD_(bal_precip_tot, 0, 1) LD_(bal_rnoff_tot, 0, 1) LD_(bal_evap_tot, 0, 1) LD_(bal_radbalsum, 0, 1)
-      LD_(ssnow_gammzz, 0, 1)
-      LF_(sum_flux_sumpn, 0, 1) LF_(sum_flux_sumrp, 0, 1) LF_(sum_flux_sumrpw, 0, 1) LF_(sum_flux_sumrpr, 0, 1)
-      LF_(sum_flux_sumrs, 0, 1) LF_(sum_flux_sumrd, 0, 1) LF_(sum_flux_dsumpn, 0, 1) LF_(sum_flux_dsumrp, 0, 1)
-      LF_(sum_flux_dsumrd, 0, 1)
+      LATE_REAL(LF_) LATE_FP64(LD_) LATE_SUMS(LF_)
 #undef LF_
 #undef LD_
     }
@@ -439,36 +464,24 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
 #undef X
     }
   };
-  // (STAGE) values that the leaf iteration does not read, in LDS through it
+  // (resident) values that the leaf iteration does not read, in their slots through it
   auto parked = [&](auto &&move) {
-    int n = LateStage<R>::PARK0;
-    move(T.ssnow_wbtot1[0], n++);
-    move(T.ssnow_wbtot2[0], n++);
-    move(T.ssnow_wb_lake[0], n++);
-    move(T.ssnow_snage[0], n++);
-    move(T.ssnow_ssdnn[0], n++);
-    move(T.rad_albedo[0], n++);
-    move(T.rad_albedo[1], n++);
-    move(T.veg_vlai[0], n++);
-    if constexpr (sizeof(R) == 8) {
-      move(T.met_fsd[0], n++);
-      move(T.met_fsd[1], n++);
-      move(T.met_precip[0], n++);
-      move(T.met_precip_sn[0], n++);
-      move(T.ssnow_otss[0], n++);
-      move(T.rad_qcan[2], n++);
-      move(T.rad_qcan[3], n++);
-      move(T.rad_flws[0], n++);
-    }
+    int n = Late::PARK0;
+#define MOVE_(id, k0, k1) \
+  { _Pragma("unroll") for (int k = k0; k < k1; k++) move(T.id[k], n++); }
+    PARKED(MOVE_)
+    if constexpr (sizeof(R) == 8) { PARKED_FP64(MOVE_) }
+#undef MOVE_
   };
-  auto unpark = [&]() { parked([&](R &x, int n) { x = late_lds.f[LateStage<R>::LANES * n]; }); };
   auto settled = [&]() {
     written(std::integral_constant<int, FIELD_SETTLED>{});
-    if constexpr (STAGE) parked([&](R &x, int n) { late_lds.f[LateStage<R>::LANES * n] = x; });
+    if constexpr (!FULL) parked([&](R &x, int n) { late_lds.f[L * n] = x; });
   };
   auto late = [&]() {
     if constexpr (FULL) {
-      __asm__ __volatile__("" ::: "memory");  // fresh reads, as below
+      // fresh reads: nothing has written these since the gather, and the
+      // compiler must not keep the gather's values live to reuse them
+      __asm__ __volatile__("" ::: "memory");
 #ifdef __HIP_DEVICE_COMPILE__
       asm volatile("" : "+s"(F));
 #endif
@@ -479,54 +492,15 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
       written(std::integral_constant<int, FIELD_CANOPY>{});
     }
     if constexpr (!FULL) {
-      using DT = typename DevT<R, 'F'>::type;
-#define LDS_(id, n) \
-  { _Pragma("unroll") for (int k = 0; k < n; k++) T.id[k] = ld<DT>(F[CABLE_F_##id], (int64_t)k * mp, t); }
-#define LDD_(id, n) \
-  { _Pragma("unroll") for (int k = 0; k < n; k++) T.id[k] = ld<double>(F[CABLE_F_##id], (int64_t)k * mp, t); }
-      // a fresh read: nothing has written these since the gather, and the
-      // compiler must not keep the gather's values live to reuse them
       __asm__ __volatile__("" ::: "memory");
-      if constexpr (STAGE) {
-        int n = 0, m = 0;
+      int n = 0, m = 0;
 #define LF_(id, k0, k1) \
-  { _Pragma("unroll") for (int k = k0; k < k1; k++) T.id[k] = late_lds.f[LateStage<R>::LANES * n++]; }
+  { _Pragma("unroll") for (int k = k0; k < k1; k++) T.id[k] = late_lds.f[L * n++]; }
 #define LD_(id, k0, k1) \
-  { _Pragma("unroll") for (int k = k0; k < k1; k++) T.id[k] = late_lds.d[LateStage<R>::LANES * m++]; }
-        LF_(ssnow_tgg, 1, 6) LF_(ssnow_tggsn, 1, 3) LF_(ssnow_smass, 0, 3) LF_(ssnow_ssdn, 0, 3) LF_(bgc_cplant, 0, 3)
-        LF_(bgc_csoil, 0, 2)
-        LD_(ssnow_wb, 1, 6) LD_(ssnow_wbice, 1, 6) LD_(drv_owb, 0, 1) LD_(bal_ebal_tot, 0, 1) LD_(bal_wbal_tot, 0, 1)
-        LD_(bal_precip_tot, 0, 1) LD_(bal_rnoff_tot, 0, 1) LD_(bal_evap_tot, 0, 1) LD_(bal_radbalsum, 0, 1)
-        LD_(ssnow_gammzz, 0, 1)
-#undef LF_
+  { _Pragma("unroll") for (int k = k0; k < k1; k++) T.id[k] = late_lds.d[L * m++]; }
+      LATE_REAL(LF_) LATE_FP64(LD_)
 #undef LD_
-        unpark();
-        return;
-      }
-#define LDL_(T_, id, k0, n) \
-  { _Pragma("unroll") for (int k = k0; k < n; k++) T.id[k] = ld<T_>(F[CABLE_F_##id], (int64_t)k * mp, t); }
-      LDL_(DT, ssnow_tgg, 1, 6) LDL_(DT, ssnow_tggsn, 1, 3) LDL_(double, ssnow_wb, 1, 6)
-      LDL_(double, ssnow_wbice, 1, 6)
-#undef LDL_
-      // values the canopy reads only before its stability iterations and
-      // soil, snow and the balances read again: the shortwave forcing, the
-      // precipitation and its snow part, and the step's starting surface
-      // temperature (otss, which the step sets from the stored tss).  FP64
-      // only: the FP32 kernel's register allocation spills more with it
-      if constexpr (sizeof(R) == 8) {
-          const R fsd = ld<DT>(F[CABLE_F_met_fsd], a.foff, t), pr = ld<DT>(F[CABLE_F_met_precip], a.foff, t);
-        T.met_fsd[0] = fsd;
-        T.met_fsd[1] = fsd;
-        T.met_precip[0] = pr;
-        T.met_precip_sn[0] = (T.met_tk[0] <= R(273.16)) ? pr : R(0.0);
-        T.ssnow_otss[0] = ld<DT>(F[CABLE_F_ssnow_tss], 0, t);
-      }
-      LDS_(ssnow_smass, 3) LDS_(ssnow_ssdn, 3) LDS_(bgc_cplant, 3) LDS_(bgc_csoil, 2)
-      LDD_(drv_owb, 1) LDD_(bal_ebal_tot, 1) LDD_(bal_wbal_tot, 1) LDD_(bal_precip_tot, 1)
-      LDD_(bal_rnoff_tot, 1) LDD_(bal_evap_tot, 1) LDD_(bal_radbalsum, 1)
-      T.ssnow_gammzz[0] = ld<double>(F[CABLE_F_ssnow_gammzz], 0, t);
-#undef LDS_
-#undef LDD_
+      parked([&](R &x, int q) { x = late_lds.f[L * q]; });
     }
   };
   if constexpr (MODE == MODE_CAPTURE) {
@@ -541,32 +515,21 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
       for (int c = 0; c < mlp::NOUT; c++) S.pred[c] = a.pred[t * mlp::NOUT + c];
     }
   }
-  // the offline driver's running carbon sums (driver mode): the resident
-  // run reads the previous step's sums only after soil and snow
+  // the offline driver's running carbon sums (every resident step is the
+  // driver's): the previous step's are read only after soil and snow
   auto tail = [&]() {
-    if constexpr (STAGE) {  // (every resident step is the driver's)
-      int n = LateStage<R>::SUM0;
-      for (R *x : {T.sum_flux_sumpn, T.sum_flux_sumrp, T.sum_flux_sumrpw, T.sum_flux_sumrpr, T.sum_flux_sumrs,
-                   T.sum_flux_sumrd, T.sum_flux_dsumpn, T.sum_flux_dsumrp, T.sum_flux_dsumrd})
-        *x = late_lds.f[LateStage<R>::LANES * n++];
-    } else if constexpr (!FULL) {
-      if (a.driver) {
-          using DT = typename DevT<R, 'F'>::type;
-        __asm__ __volatile__("" ::: "memory");
-#define LDF_(id) T.id[0] = ld<DT>(F[CABLE_F_##id], 0, t);
-        LDF_(sum_flux_sumpn) LDF_(sum_flux_sumrp) LDF_(sum_flux_sumrpw) LDF_(sum_flux_sumrpr)
-        LDF_(sum_flux_sumrs) LDF_(sum_flux_sumrd) LDF_(sum_flux_dsumpn) LDF_(sum_flux_dsumrp)
-        LDF_(sum_flux_dsumrd)
-#undef LDF_
-      }
+    if constexpr (!FULL) {
+      int n = Late::SUM0;
+      LATE_SUMS(LF_)
     }
   };
+#undef LF_
   auto stash = [&]() {
-    if constexpr (STAGE) {
+    if constexpr (!FULL) {
 #pragma unroll
-      for (int q = 0; q < LateStage<R>::PARK0; q++) late_lds.f[LateStage<R>::LANES * q] = lf[q];
+      for (int q = 0; q < Late::PARK0; q++) late_lds.f[L * q] = lf[q];
 #pragma unroll
-      for (int q = 0; q < LateStage<R>::ND; q++) late_lds.d[LateStage<R>::LANES * q] = ld_[q];
+      for (int q = 0; q < Late::ND; q++) late_lds.d[L * q] = ld_[q];
     }
   };
   // the previous-step canopy state the surrogate's features read (written
@@ -633,6 +596,53 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
   }
 }
 
+// One class-table value in a workgroup's tables: in the working type, and in FP64
+// beside them the columns that an FP32 step reads so (ClassRows).
+template <class V>
+CBM_HD void put_veg(int i, double x, V *v, double *vd) {
+  v[i] = (V)x;
+  if constexpr (sizeof(V) == 4) {
+    const int c = i % VC_N - VC_fes_cor;
+    if (c >= 0 && c < NVEGD) vd[i / VC_N * NVEGD + c] = x;
+  }
+}
+template <class V>
+CBM_HD void put_soil(int i, double x, V *s, double *sd) {
+  s[i] = (V)x;
+  if constexpr (sizeof(V) == 4) sd[i] = x;
+}
+// the i-th derived column from the vegetation table there
+template <class R, class V>
+CBM_HD V derived_column(int i, const V *v) {
+  return Stepper<R, false, true, MODE_PLAIN, V, true>::derived(i % VX_N, [&](int c) { return (R)v[i / VX_N * VC_N + c]; });
+}
+
+#ifdef __HIP_DEVICE_COMPILE__
+typedef const __attribute__((address_space(4))) StepArgs *StepList;
+#else
+typedef const StepArgs *StepList;
+#endif
+// `nsteps` plain resident steps of a tile, one after the other; returns the
+// leaf passes
+template <class R, class V = R>
+CBM_HD int run_tile(StepList args, int nsteps, int64_t tile, bool live, const V *vtab, const V *stab, LateStage<R> late,
+                    const V *xtab, const double *vdtab, const double *sdtab) {
+  TileOut<MODE_PLAIN, false> o;
+  int passes = 0;
+  for (int k = 0; k < nsteps; k++, args++) {
+    // nothing of a step is kept for the next: the arguments are read again
+    // and the tile's offsets formed again, which the compiler would hold in
+    // registers through every step
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+s"(args), "+v"(tile) : : "memory");
+#endif
+    step_tile<R, false, true, MODE_PLAIN, false, true, V>(*(const StepArgs *)args, tile, vtab, stab, o, late, xtab,
+                                                          vdtab, sdtab, NoTables(), live);
+    passes += o.passes;
+  }
+  return passes;
+}
+
 // CONS: also form the workgroup's sums for the driver's consistency check
 // (a separate instantiation: the check's code costs the plain step 2-3% even
 // when it is switched off at run time)
@@ -673,23 +683,15 @@ cbm_kernel(StepArgs a) {
 #pragma unroll
       for (int q = 0; q < (NV + B - 1) / B; q++) {
         const int i = threadIdx.x + q * B;
-        if (i < NV) lds_v[i] = (V)tv[q];
-        if constexpr (sizeof(V) == 4) {
-          const int c = i % VC_N - VC_fes_cor;
-          if (i < NV && c >= 0 && c < NVEGD) lds_vd[i / VC_N * NVEGD + c] = tv[q];
-        }
+        if (i < NV) put_veg(i, tv[q], lds_v, lds_vd);
       }
 #pragma unroll
       for (int q = 0; q < (NS + B - 1) / B; q++) {
         const int i = threadIdx.x + q * B;
-        if (i < NS) lds_s[i] = (V)ts[q];
-        if constexpr (sizeof(V) == 4)
-          if (i < NS) lds_sd[i] = ts[q];
+        if (i < NS) put_soil(i, ts[q], lds_s, lds_sd);
       }
       lds_barrier();
-      for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B)
-        lds_x[i] = Stepper<R, FULL, TABLES, MODE, V, true>::derived(
-            i % VX_N, [&](int c) { return (R)lds_v[i / VX_N * VC_N + c]; });
+      for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B) lds_x[i] = derived_column<R>(i, lds_v);
       lds_barrier();
     }
   };
@@ -713,25 +715,9 @@ cbm_kernel(StepArgs a) {
     // stage the tables once.  A day (48 steps) of 262,144 tiles in FP64 15.1 ->
     // 13.1 ms, of 1,048,576 in mixed precision 18.1 -> 16.9 ms, of 20,011 tiles
     // 2.58 -> 2.15 ms; 12 steps a launch gave two thirds of it.
-    const int nsteps = a.nsteps;
     tables();
-#ifdef __HIP_DEVICE_COMPILE__
-    auto args = (const __attribute__((address_space(4))) StepArgs *)(uintptr_t)a.steps;
-#else
-    const StepArgs *args = a.steps;
-#endif
-    int64_t tile = live ? t : mp - 1;
-    for (int k = 0; k < nsteps; k++, args++) {
-      // nothing of a step is kept for the next: the arguments are read again
-      // and the tile's offsets formed again, which the compiler would hold in
-      // registers through every step
-#ifdef __HIP_DEVICE_COMPILE__
-      asm volatile("" : "+s"(args), "+v"(tile) : : "memory");
-#endif
-      step_tile<R, FULL, TABLES, MODE, CONS, true, V>(*(const StepArgs *)args, tile, lds_v, lds_s, o, late, lds_x,
-                                                      lds_vd, lds_sd, NoTables(), live);
-      passes += o.passes;
-    }
+    passes = run_tile<R>((StepList)(uintptr_t)a.steps, a.nsteps, live ? t : mp - 1, live, lds_v, lds_s, late, lds_x,
+                         lds_vd, lds_sd);
   } else {
     step_tile<R, FULL, TABLES, MODE, CONS, true, V>(a, live ? t : mp - 1, lds_v, lds_s, o, late, lds_x, lds_vd,
                                                     lds_sd, tables, live);
