@@ -596,20 +596,24 @@ CBM_HD void step_tile(const StepArgs &a, int64_t t, const std::common_type_t<V> 
   }
 }
 
-// One class-table value in a workgroup's tables: in the working type, and in FP64
-// beside them the columns that an FP32 step reads so (ClassRows).
+// One class-table value (where there is an i-th) in a workgroup's tables: in the
+// working type, and in FP64 beside them the columns that an FP32 step reads so
+// (ClassRows).
 template <class V>
 CBM_HD void put_veg(int i, double x, V *v, double *vd) {
-  v[i] = (V)x;
+  constexpr int N = NVEGCLASS * VC_N;
+  if (i < N) v[i] = (V)x;
   if constexpr (sizeof(V) == 4) {
     const int c = i % VC_N - VC_fes_cor;
-    if (c >= 0 && c < NVEGD) vd[i / VC_N * NVEGD + c] = x;
+    if (i < N && c >= 0 && c < NVEGD) vd[i / VC_N * NVEGD + c] = x;
   }
 }
 template <class V>
 CBM_HD void put_soil(int i, double x, V *s, double *sd) {
-  s[i] = (V)x;
-  if constexpr (sizeof(V) == 4) sd[i] = x;
+  constexpr int N = NSOILCLASS * SC_N;
+  if (i < N) s[i] = (V)x;
+  if constexpr (sizeof(V) == 4)
+    if (i < N) sd[i] = x;
 }
 // the i-th derived column from the vegetation table there
 template <class R, class V>
@@ -683,12 +687,12 @@ cbm_kernel(StepArgs a) {
 #pragma unroll
       for (int q = 0; q < (NV + B - 1) / B; q++) {
         const int i = threadIdx.x + q * B;
-        if (i < NV) put_veg(i, tv[q], lds_v, lds_vd);
+        put_veg(i, tv[q], lds_v, lds_vd);
       }
 #pragma unroll
       for (int q = 0; q < (NS + B - 1) / B; q++) {
         const int i = threadIdx.x + q * B;
-        if (i < NS) put_soil(i, ts[q], lds_s, lds_sd);
+        put_soil(i, ts[q], lds_s, lds_sd);
       }
       lds_barrier();
       for (int i = threadIdx.x; i < NVEGCLASS * VX_N; i += B) lds_x[i] = derived_column<R>(i, lds_v);
