@@ -334,44 +334,47 @@ void on_threads(int device, size_t bytes, F &&f) {
   for (auto &t : th) t.join();
 }
 
-// fill(b0, b1) packs bytes [b0, b1) of the staging buffer; `bytes` of it go
+// fill(b0, b1) packs bytes [b0, b1) of the staging buffer; [from, end) of it go
 // to its device twin (`copy`) on the context's stream
 template <class F>
-hipError_t stage_up(cable_gpu_ctx *c, size_t bytes, bool copy, F &&fill) {
+hipError_t stage_up(cable_gpu_ctx *c, size_t from, size_t end, bool copy, F &&fill) {
   constexpr size_t PER = XFER_UNIT / XFER_PIECE;
-  const size_t units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
+  const size_t bytes = end - from, units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
   std::vector<std::atomic<size_t>> packed(units);
   for (auto &u : packed) u = 0;
   std::atomic<int> err(hipSuccess);
   on_threads(c->device, bytes, [&](size_t q) {
     const size_t u = q / PER, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
-    fill(q * XFER_PIECE, std::min(bytes, (q + 1) * XFER_PIECE));
+    fill(from + q * XFER_PIECE, from + std::min(bytes, (q + 1) * XFER_PIECE));
     if (packed[u].fetch_add(1) + 1 == (u1 - u0 + XFER_PIECE - 1) / XFER_PIECE && copy) {
-      const hipError_t e = hipMemcpyAsync(c->d_stage + u0, c->h_stage + u0, u1 - u0, hipMemcpyHostToDevice, c->stream);
+      const hipError_t e = hipMemcpyAsync(c->d_stage + from + u0, c->h_stage + from + u0, u1 - u0, hipMemcpyHostToDevice,
+                                          c->stream);
       if (e != hipSuccess) err = e;
     }
   });
   return (hipError_t)err.load();
 }
 
-// host arrays one after the other in the staging buffer, each at a multiple
-// of 256 bytes, and the same on the device
+constexpr size_t align_up(size_t n) { return (n + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN; }
+
+// host arrays one after the other in [from, end) of the staging buffer, each at
+// a multiple of 256 bytes, and the same on the device
 struct StageList {
   struct Seg {
     const void *host;
     size_t off, bytes;
   };
   std::vector<Seg> segs;
-  size_t bytes = 0;
+  size_t from = 0, end = 0;
   // the array's offset
   size_t add(const void *host, size_t n) {
-    const size_t off = bytes;
+    const size_t off = end;
     segs.push_back({host, off, n});
-    bytes += (n + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN;
+    end += align_up(n);
     return off;
   }
   hipError_t up(cable_gpu_ctx *c) const {
-    return stage_up(c, bytes, true, [&](size_t b0, size_t b1) {
+    return stage_up(c, from, end, true, [&](size_t b0, size_t b1) {
       for (const Seg &g : segs) {
         const size_t l0 = std::max(b0, g.off), l1 = std::min(b1, g.off + g.bytes);
         if (l0 < l1) memcpy(c->h_stage + l0, (const unsigned char *)g.host + (l0 - g.off), l1 - l0);
@@ -380,6 +383,17 @@ struct StageList {
   }
 };
 
+// the context's first n events
+hipError_t ensure_events(cable_gpu_ctx *c, size_t n) {
+  while (c->xev.size() < n) {
+    hipEvent_t ev;
+    const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+    c->xev.push_back(ev);
+  }
+  return hipSuccess;
+}
+
 // the device twin's `bytes` come back (`copy`) on the context's stream and
 // drain(b0, b1) unpacks them; ends when all has arrived
 template <class F>
@@ -387,15 +401,10 @@ hipError_t stage_down(cable_gpu_ctx *c, size_t bytes, bool copy, F &&drain) {
   const size_t units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
   hipError_t e = hipSuccess;
   if (copy && units > 1) {
+    e = ensure_events(c, units);
     for (size_t u = 0; u < units && e == hipSuccess; u++) {
       const size_t u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
-      if (c->xev.size() <= u) {
-        hipEvent_t ev;
-        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-        if (e == hipSuccess) c->xev.push_back(ev);
-      }
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(c->h_stage + u0, c->d_stage + u0, u1 - u0, hipMemcpyDeviceToHost, c->stream);
+      e = hipMemcpyAsync(c->h_stage + u0, c->d_stage + u0, u1 - u0, hipMemcpyDeviceToHost, c->stream);
       if (e == hipSuccess) e = hipEventRecord(c->xev[u], c->stream);
     }
   } else {
@@ -446,7 +455,7 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
       return fail(CABLE_E_ARG, "%s: bad host type %d (entry %d)", who, types[k], k);
     const FieldMeta &f = kFields[ids[k]];
     tab[k] = {c->dev[ids[k]], off, f.n, (int)dev_elem(f, c->precision)};
-    off += (field_bytes(c, ids[k]) + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN;
+    off += align_up(field_bytes(c, ids[k]));
   }
   if (n == 0) return CABLE_OK;
   if (const int r = ensure_stage(c, off)) return r;
@@ -473,7 +482,7 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
   const dim3 grid((unsigned)std::min<int64_t>(1024, (c->mp + 255) / 256), (unsigned)n);
   if (up) {
     c->touched = true;
-    const hipError_t e = stage_up(c, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, true); });
+    const hipError_t e = stage_up(c, 0, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, true); });
     if (e != hipSuccess) {
       (void)hipStreamSynchronize(c->stream);
       return fail(CABLE_E_HIP, "%s: %s", who, hipGetErrorString(e));
@@ -1067,9 +1076,14 @@ __device__ inline R met_svp(R tk) {
   return pow(R(10.0), ewlog4);
 }
 
-// (12 steps of 131,071 tiles: 1.2 ms, 2.1 ms in 13 buffers allocated and
-// copied one by one from pageable memory)
-constexpr size_t MET_STAGE = 64 << 20;
+// Half of a met window's staging buffer: bound by the host's copies into it, and
+// in a new context by the first touch of its pages (0.06 ms a MiB on eight
+// threads).  12 steps of 131,071 tiles (48 MiB) 1.2 ms, in a new context 3.4 ms;
+// in one buffer of up to 64 MiB 1.1 and 4.8 ms, in halves of 4 MiB 1.3 and 3.3,
+// of 16 MiB 1.2 and 4.5; in 13 buffers allocated and copied one by one
+// from pageable memory 2.0 and 8.0 ms (2.5 where the runtime had the memory of
+// closed contexts at hand, here 4.1).
+constexpr size_t MET_STAGE = 8 << 20;
 
 struct MetArgs {
   const float *swdown, *lwdown, *tair, *qair, *wind, *wind_e, *psurf, *rainf;
@@ -1316,7 +1330,7 @@ int cable_gpu_synth_forcing(cable_gpu_ctx *c, int k_first, int nsteps, uint64_t 
   StageList in;
   in.add(t0, sizeof(double) * mp);
   const size_t lat_off = in.add(lat, sizeof(double) * mp);
-  if (const int r = ensure_stage(c, in.bytes)) return r;
+  if (const int r = ensure_stage(c, in.end)) return r;
   const hipError_t e = in.up(c);
   if (e != hipSuccess) {
     (void)hipStreamSynchronize(c->stream);
@@ -1374,28 +1388,40 @@ int cable_gpu_set_met(cable_gpu_ctx *c, int k_first, int nsteps, double dels, co
     for (int i = 0; i < 8; i++) HIPCHECK(hipMalloc(&c->forc[i], bytes));
   }
   // the met variables to the device in the caller's tile order, through the
-  // staging buffer: as many steps at a time as MET_STAGE bytes hold
+  // staging buffer: what does not change with the steps, then the steps in
+  // chunks through the buffer's two halves in turn, so that the host packs one
+  // while the other is copied
   const float *const vars[8] = {m->swdown, m->lwdown, m->tair, m->qair, m->wind, m->wind_e, m->psurf, m->rainf};
   size_t per_step = 0;
   for (const float *v : vars) per_step += v ? sizeof(float) * mp : 0;
   const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)nsteps, MET_STAGE / per_step));
-  for (int s0 = 0; s0 < nsteps; s0 += chunk) {
+  StageList fixed;
+  const size_t lat = fixed.add(m->latitude, sizeof(double) * mp);
+  const size_t elev = m->elevation ? fixed.add(m->elevation, sizeof(double) * mp) : 0;
+  const size_t hods = fixed.add(hod.data(), sizeof(double) * hod.size());
+  const size_t doys = fixed.add(doy.data(), sizeof(double) * doy.size());
+  size_t half = 0;
+  for (const float *v : vars) half += v ? align_up(sizeof(float) * (size_t)chunk * mp) : 0;
+  if (const int r = ensure_stage(c, fixed.end + (chunk < nsteps ? 2 : 1) * half)) return r;
+  c->nsteps_forc = 0;  // the window there is overwritten from here on
+  hipError_t e = ensure_events(c, 2);
+  if (e == hipSuccess) e = fixed.up(c);
+  for (int s0 = 0, q = 0; s0 < nsteps && e == hipSuccess; s0 += chunk, q++) {
     const int ns = std::min(chunk, nsteps - s0);
     StageList in;
-    const size_t lat = in.add(m->latitude, sizeof(double) * mp);
-    const size_t elev = m->elevation ? in.add(m->elevation, sizeof(double) * mp) : 0;
-    const size_t hods = in.add(hod.data() + s0, sizeof(double) * (size_t)ns);
-    const size_t doys = in.add(doy.data() + s0, sizeof(double) * (size_t)ns);
+    in.from = in.end = fixed.end + (size_t)(q & 1) * half;
     size_t at[8];
     for (int v = 0; v < 8; v++)
       at[v] = vars[v] ? in.add(vars[v] + (size_t)s0 * mp, sizeof(float) * (size_t)ns * mp) : 0;
-    if (const int r = ensure_stage(c, in.bytes)) return r;
-    hipError_t e = in.up(c);
+    if (q > 1) e = hipEventSynchronize(c->xev[q & 1]);
+    if (e == hipSuccess) e = in.up(c);
+    if (e == hipSuccess) e = hipEventRecord(c->xev[q & 1], c->stream);
+    if (e != hipSuccess) break;
     auto var = [&](int v) { return vars[v] ? (const float *)(c->d_stage + at[v]) : nullptr; };
     const MetArgs a = {var(0), var(1), var(2), var(3), var(4), var(5), var(6), var(7), c->d_order,
                        m->elevation ? (const double *)(c->d_stage + elev) : nullptr,
-                       (const double *)(c->d_stage + lat), (const double *)(c->d_stage + hods),
-                       (const double *)(c->d_stage + doys), m->tair_offset, m->psurf_scale, m->rainf_scale,
+                       (const double *)(c->d_stage + lat), (const double *)(c->d_stage + hods) + s0,
+                       (const double *)(c->d_stage + doys) + s0, m->tair_offset, m->psurf_scale, m->rainf_scale,
                        m->qair_is_rh};
     const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)ns);
     auto go = [&](auto zero) {
@@ -1405,15 +1431,13 @@ int cable_gpu_set_met(cable_gpu_ctx *c, int k_first, int nsteps, double dels, co
       hipLaunchKernelGGL(met_kernel<R>, grid, dim3(256), 0, c->stream, c->mp, a, f[0], f[1], f[2], f[3], f[4], f[5],
                          f[6], f[7]);
     };
-    if (e == hipSuccess) {
-      if (c->precision == CABLE_PREC_MIXED) go(0.0f);
-      else go(0.0);
-      e = hipGetLastError();
-    }
-    const hipError_t w = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = w;
-    if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString(e));
+    if (c->precision == CABLE_PREC_MIXED) go(0.0f);
+    else go(0.0);
+    e = hipGetLastError();
   }
+  const hipError_t w = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = w;
+  if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString(e));
   const int ids[8] = {CABLE_F_met_fsd, CABLE_F_met_fld, CABLE_F_met_tk, CABLE_F_met_qv,
                       CABLE_F_met_ua, CABLE_F_met_pmb, CABLE_F_met_precip, CABLE_F_met_coszen};
   std::vector<void *> tab = c->dev;
