@@ -21,6 +21,7 @@
 
 #include "../../include/cable_gpu.h"
 #include "cbm_kernel.h"
+#include "staging.h"
 
 using namespace cbm;
 
@@ -193,15 +194,8 @@ struct cable_gpu_ctx {
 
 namespace {
 // ---- batched transfers ----
-// One entry per field of a batched transfer: the field's device array, its
-// offset in the staging buffer, its rows of mp values and a value's bytes.
-struct XferEntry {
-  void *dev;
-  unsigned long long off;
-  int rows, bytes;
-};
-constexpr size_t XFER_TABLE_BYTES = sizeof(XferEntry) * CABLE_NFIELDS;
-constexpr size_t XFER_ALIGN = 256;
+using XferEntry = staging::Entry;
+using staging::align_up;
 
 // dst(:, r) = src(perm, r)
 template <class T>
@@ -234,7 +228,7 @@ __global__ void __launch_bounds__(256) xfer_kernel(const XferEntry *__restrict__
       permute_rows((uint32_t *)dst, (const uint32_t *)src, perm, mp, e.rows);
     return;
   }
-  // both sides are aligned to 256 bytes: 16 bytes at a time, then the rest
+  // both sides are aligned to 256 bytes (staging.h): 16 bytes at a time, then the rest
   const int64_t words = (int64_t)e.rows * mp * (e.bytes / 4), wide = words / 4;
   const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = i0; i < wide; i += stride) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
@@ -300,38 +294,12 @@ int ensure_stage(cable_gpu_ctx *c, size_t bytes) {
   return CABLE_OK;
 }
 
-// The staging buffer is packed (unpacked) in pieces on up to eight threads,
-// one per XFER_THREAD bytes (starting one costs as much as it saves below: 11
-// fields of 8,000 tiles down, 0.7 MB, 67 us with one thread, 76 with three),
-// and copied in units, each when its pieces are packed or before they are
-// unpacked, so that the copies and the host's work overlap: every field of
-// 49,149 tiles up in 3.9 ms (152 MB; 4.9 packed first), down in 2.9 ms (3.6).
-// Units of 1 and 2 MiB were slower (4.7 and 4.1 ms up), of 8 MiB faster for
-// this and slower for small batches.
-constexpr size_t XFER_THREAD = 1 << 20, XFER_PIECE = 512 << 10, XFER_UNIT = 4 << 20;
+constexpr size_t XFER_PIECE = 512 << 10, XFER_UNIT = staging::UNIT;
 
-// f(piece) for every piece of `bytes`
+// f(piece) for every piece of `bytes`, on the host's threads
 template <class F>
-void on_threads(int device, size_t bytes, F &&f) {
-  const size_t pieces = (bytes + XFER_PIECE - 1) / XFER_PIECE;
-  std::atomic<size_t> next(0);
-  auto run = [&]() {
-    for (size_t q; (q = next.fetch_add(1)) < pieces;) f(q);
-  };
-  const unsigned nt = (unsigned)std::min<size_t>(
-      {8, pieces, bytes / XFER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
-  std::vector<std::thread> th;
-  for (unsigned t = 1; t < nt; t++) {
-    try {
-      th.emplace_back([&]() {
-        if (hipSetDevice(device) == hipSuccess) run();
-      });
-    } catch (...) {  // no more threads: those there do the work
-      break;
-    }
-  }
-  run();
-  for (auto &t : th) t.join();
+void on_threads(const cable_gpu_ctx *c, size_t bytes, F &&f) {
+  staging::on_threads(bytes, XFER_PIECE, [&]() { return hipSetDevice(c->device) == hipSuccess; }, f);
 }
 
 // fill(b0, b1) packs bytes [b0, b1) of the staging buffer; [from, end) of it go
@@ -343,7 +311,7 @@ hipError_t stage_up(cable_gpu_ctx *c, size_t from, size_t end, bool copy, F &&fi
   std::vector<std::atomic<size_t>> packed(units);
   for (auto &u : packed) u = 0;
   std::atomic<int> err(hipSuccess);
-  on_threads(c->device, bytes, [&](size_t q) {
+  on_threads(c, bytes, [&](size_t q) {
     const size_t u = q / PER, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
     fill(from + q * XFER_PIECE, from + std::min(bytes, (q + 1) * XFER_PIECE));
     if (packed[u].fetch_add(1) + 1 == (u1 - u0 + XFER_PIECE - 1) / XFER_PIECE && copy) {
@@ -354,8 +322,6 @@ hipError_t stage_up(cable_gpu_ctx *c, size_t from, size_t end, bool copy, F &&fi
   });
   return (hipError_t)err.load();
 }
-
-constexpr size_t align_up(size_t n) { return (n + XFER_ALIGN - 1) / XFER_ALIGN * XFER_ALIGN; }
 
 // host arrays one after the other in [from, end) of the staging buffer, each at
 // a multiple of 256 bytes, and the same on the device
@@ -416,7 +382,7 @@ hipError_t stage_down(cable_gpu_ctx *c, size_t bytes, bool copy, F &&drain) {
     return e;
   }
   std::atomic<int> err(hipSuccess);
-  on_threads(c->device, bytes, [&](size_t q) {
+  on_threads(c, bytes, [&](size_t q) {
     if (copy && units > 1) {
       const hipError_t w = hipEventSynchronize(c->xev[q * XFER_PIECE / XFER_UNIT]);
       if (w != hipSuccess) {
@@ -447,7 +413,7 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
   const char *who = up ? "cable_gpu_upload_fields" : "cable_gpu_download_fields";
   if (n > CABLE_NFIELDS) return fail(CABLE_E_ARG, "%s: %d fields (at most %d)", who, n, CABLE_NFIELDS);
   std::vector<XferEntry> tab(n);
-  size_t off = XFER_TABLE_BYTES;
+  size_t off = staging::TABLE_BYTES;
   for (int k = 0; k < n; k++) {
     if (ids[k] < 0 || ids[k] >= CABLE_NFIELDS || !hosts[k])
       return fail(CABLE_E_ARG, "%s: bad field %d (entry %d)", who, ids[k], k);

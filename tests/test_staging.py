@@ -1,0 +1,29 @@
+"""The staging buffer's layout and the sharing of its packing
+(cable_amd/csrc/staging.h), on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not found")
+
+
+@pytest.fixture(scope="module")
+def lines(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("staging") / "s")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", os.path.join(HERE, "host_staging.cpp"), "-o", exe],
+                   check=True, capture_output=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout
+    return [(x.split()[0], [int(v) for v in x.split()[1:]]) for x in out.splitlines()]
+
+
+def test_every_array_starts_at_the_alignment(lines):
+    assert dict(lines)["offsets"] == [0, 0, 0, 0]
+
+
+def test_every_piece_is_handed_out_once(lines):
+    got = [v for k, v in lines if k == "pieces"]
+    assert len(got) == 10 and all(n == once for n, once in got)
