@@ -294,27 +294,26 @@ int ensure_stage(cable_gpu_ctx *c, size_t bytes) {
   return CABLE_OK;
 }
 
-constexpr size_t XFER_PIECE = 512 << 10, XFER_UNIT = staging::UNIT;
+constexpr size_t XFER_UNIT = staging::UNIT;
 
-// f(piece) for every piece of `bytes`, on the host's threads
+// f(b0, b1) for every piece of `bytes`, on the host's threads
 template <class F>
 void on_threads(const cable_gpu_ctx *c, size_t bytes, F &&f) {
-  staging::on_threads(bytes, XFER_PIECE, [&]() { return hipSetDevice(c->device) == hipSuccess; }, f);
+  staging::on_threads(bytes, [&]() { return hipSetDevice(c->device) == hipSuccess; }, f);
 }
 
 // fill(b0, b1) packs bytes [b0, b1) of the staging buffer; [from, end) of it go
 // to its device twin (`copy`) on the context's stream
 template <class F>
 hipError_t stage_up(cable_gpu_ctx *c, size_t from, size_t end, bool copy, F &&fill) {
-  constexpr size_t PER = XFER_UNIT / XFER_PIECE;
   const size_t bytes = end - from, units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
   std::vector<std::atomic<size_t>> packed(units);
   for (auto &u : packed) u = 0;
   std::atomic<int> err(hipSuccess);
-  on_threads(c, bytes, [&](size_t q) {
-    const size_t u = q / PER, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
-    fill(from + q * XFER_PIECE, from + std::min(bytes, (q + 1) * XFER_PIECE));
-    if (packed[u].fetch_add(1) + 1 == (u1 - u0 + XFER_PIECE - 1) / XFER_PIECE && copy) {
+  on_threads(c, bytes, [&](size_t b0, size_t b1) {
+    const size_t u = b0 / XFER_UNIT, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
+    fill(from + b0, from + b1);
+    if (packed[u].fetch_add(b1 - b0) + (b1 - b0) == u1 - u0 && copy) {
       const hipError_t e = hipMemcpyAsync(c->d_stage + from + u0, c->h_stage + from + u0, u1 - u0, hipMemcpyHostToDevice,
                                           c->stream);
       if (e != hipSuccess) err = e;
@@ -382,15 +381,15 @@ hipError_t stage_down(cable_gpu_ctx *c, size_t bytes, bool copy, F &&drain) {
     return e;
   }
   std::atomic<int> err(hipSuccess);
-  on_threads(c, bytes, [&](size_t q) {
+  on_threads(c, bytes, [&](size_t b0, size_t b1) {
     if (copy && units > 1) {
-      const hipError_t w = hipEventSynchronize(c->xev[q * XFER_PIECE / XFER_UNIT]);
+      const hipError_t w = hipEventSynchronize(c->xev[b0 / XFER_UNIT]);
       if (w != hipSuccess) {
         err = w;
         return;
       }
     }
-    drain(q * XFER_PIECE, std::min(bytes, (q + 1) * XFER_PIECE));
+    drain(b0, b1);
   });
   if (err != hipSuccess) (void)hipStreamSynchronize(c->stream);  // the buffer is not left in use
   return (hipError_t)err.load();

@@ -1,7 +1,7 @@
 // host_staging.cpp -- cable_amd/csrc/staging.h by itself, for
 // tests/test_staging.py: prints, one line each, the offsets of a batch's arrays
-// modulo the alignment they need, and how often the pieces of a buffer of some
-// sizes were handed out.
+// modulo the alignment they need, and how the bytes of a buffer of some sizes were
+// handed out.
 #include <stdio.h>
 
 #include "../cable_amd/csrc/staging.h"
@@ -14,21 +14,27 @@ int main() {
   printf("offsets");
   for (int k = 0; k < 4; k++, off += align_up(77 * 8)) printf(" %zu", off % ALIGN);
   printf("\n");
-  // each byte once, whatever the threads
-  for (size_t bytes : {(size_t)1, (size_t)65536, (size_t)UNIT - 1, (size_t)UNIT + 1, 9 * (size_t)UNIT + 12345}) {
-    const size_t piece = 512 << 10, n = (bytes + piece - 1) / piece;
-    std::vector<std::atomic<int>> seen(n);
-    for (auto &x : seen) x = 0;
-    on_threads(bytes, piece, [] { return true; }, [&](size_t q) { seen[q]++; });
-    size_t once = 0;
-    for (auto &x : seen) once += x == 1;
-    printf("pieces %zu %zu\n", n, once);
-    // threads that cannot start leave the work to the first
-    for (auto &x : seen) x = 0;
-    on_threads(bytes, piece, [] { return false; }, [&](size_t q) { seen[q]++; });
-    once = 0;
-    for (auto &x : seen) once += x == 1;
-    printf("pieces %zu %zu\n", n, once);
+  // each byte once, whether threads start or leave the work to the first; the
+  // most threads that have a part of one aligned 2 MiB; pieces beyond their unit
+  const size_t unit = UNIT, large = 2 << 20;
+  for (size_t bytes : {(size_t)1, (size_t)65536, unit - 1, unit + 1, 4 * unit - 1, 4 * unit, 9 * unit + 12345}) {
+    for (bool starts : {true, false}) {
+      std::vector<std::atomic<int>> seen(bytes), parts(bytes / large + 1);
+      for (auto &x : seen) x = 0;
+      for (auto &x : parts) x = 0;
+      std::atomic<size_t> beyond(0);
+      on_threads(bytes, [&] { return starts; }, [&](size_t b0, size_t b1) {
+        for (size_t b = b0; b < b1; b++) seen[b]++;
+        beyond += b0 / unit != (b1 - 1) / unit;
+        for (size_t p = b0 / large; p <= (b1 - 1) / large; p++) parts[p]++;
+      });
+      size_t once = 0;
+      int most = 0;
+      for (auto &x : seen) once += x == 1;
+      for (size_t p = 0; p + 1 < parts.size() && (p + 1) * large + unit + large <= bytes; p++)
+        most = std::max(most, parts[p].load());
+      printf("pieces %zu %zu %zu %d\n", bytes, once, (size_t)beyond, bytes < 4 * unit ? 1 : most);
+    }
   }
   return 0;
 }

@@ -24,6 +24,12 @@ def test_every_array_starts_at_the_alignment(lines):
     assert dict(lines)["offsets"] == [0, 0, 0, 0]
 
 
-def test_every_piece_is_handed_out_once(lines):
+def test_every_byte_is_handed_out_once_in_pieces_within_a_unit(lines):
     got = [v for k, v in lines if k == "pieces"]
-    assert len(got) == 10 and all(n == once for n, once in got)
+    assert len(got) == 14 and all(n == once and beyond == 0 for n, once, beyond, _ in got)
+
+
+def test_a_large_buffer_is_not_shared_within_a_huge_page(lines):
+    """From 16 MiB on, but for the last 4 to 6 MiB: else the threads that touch a
+    page of a new array first wait for each other."""
+    assert all(most == 1 for k, v in lines if k == "pieces" for most in v[3:])
