@@ -282,6 +282,7 @@ size_t field_bytes(const cable_gpu_ctx *c, int id) {
 // the staging buffer and its device twin, of at least `bytes`
 int ensure_stage(cable_gpu_ctx *c, size_t bytes) {
   if (bytes <= c->stage_bytes) return CABLE_OK;
+  bytes = staging::capacity(bytes);
   HIPCHECK(hipStreamSynchronize(c->stream));
   if (c->h_stage) HIPCHECK(hipHostFree(c->h_stage));
   c->h_stage = nullptr;

@@ -36,5 +36,16 @@ int main() {
       printf("pieces %zu %zu %zu %d\n", bytes, once, (size_t)beyond, bytes < 4 * unit ? 1 : most);
     }
   }
+  // what a context of some tiles asks for in turn: its forcing's inputs, the surface
+  // fluxes and the soil (29 values), and the times it pins for them
+  for (size_t mp : {77, 1000, 4093, 20011}) {
+    size_t have = 0, pins = 0;
+    for (size_t need : {16 * mp, TABLE_BYTES + 14 * ALIGN + 29 * 8 * mp}) {
+      if (need <= have) continue;
+      have = capacity(need);
+      pins += have >= need;
+    }
+    printf("pins %zu %zu\n", mp, pins);
+  }
   return 0;
 }

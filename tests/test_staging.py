@@ -33,3 +33,7 @@ def test_a_large_buffer_is_not_shared_within_a_huge_page(lines):
     """From 16 MiB on, but for the last 4 to 6 MiB: else the threads that touch a
     page of a new array first wait for each other."""
     assert all(most == 1 for k, v in lines if k == "pieces" for most in v[3:])
+
+
+def test_a_small_context_pins_once(lines):
+    assert [v for k, v in lines if k == "pins"] == [[77, 1], [1000, 1], [4093, 1], [20011, 2]]
