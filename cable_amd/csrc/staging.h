@@ -27,12 +27,13 @@ constexpr size_t align_up(size_t n) { return (n + ALIGN - 1) / ALIGN * ALIGN; }
 constexpr size_t TABLE_BYTES = align_up(sizeof(Entry) * CABLE_NFIELDS);
 static_assert(TABLE_BYTES % ALIGN == 0 && ALIGN % 16 == 0, "the kernel's 16-byte accesses");
 
-// The size of a buffer that `need` bytes ask for: at least 1 MiB, so that a small
-// context pins once for what it sends and reads (its forcing's inputs, then the
-// first read-back with the soil: 77 tiles 0.26 ms against 0.28 to 0.6, 4,093 in FP64
-// 0.89 against 0.96).  Not more: a buffer that is given back for a larger one costs
-// a new context 0.2 ms (1 MiB) to 0.8 ms (4 MiB).
-constexpr size_t capacity(size_t need) { return std::max(need, (size_t)1 << 20); }
+// The size of a buffer that `need` bytes ask for: at least 256 KiB, so that a
+// small context pins once for what it sends and reads (its forcing's inputs, then
+// the first read-back with the soil: 77 tiles 0.2 ms against 0.25 to 0.55, 1,000
+// in FP64 0.36 against 0.43).  Not more: pinning 1 MiB takes 0.05 to 0.1 ms longer,
+// which a context that needs less pays, and a buffer given back for a larger
+// one as much again.
+constexpr size_t capacity(size_t need) { return std::max(need, (size_t)256 << 10); }
 
 // The buffer is packed (unpacked) in pieces on up to eight threads, one per
 // PER_THREAD bytes (starting one costs as much as it saves below: 11 fields of

@@ -36,4 +36,4 @@ def test_a_large_buffer_is_not_shared_within_a_huge_page(lines):
 
 
 def test_a_small_context_pins_once(lines):
-    assert [v for k, v in lines if k == "pins"] == [[77, 1], [1000, 1], [4093, 1], [20011, 2]]
+    assert [v for k, v in lines if k == "pins"] == [[77, 1], [1000, 1], [4093, 2], [20011, 2]]
