@@ -303,23 +303,27 @@ void on_threads(const cable_gpu_ctx *c, size_t bytes, F &&f) {
   staging::on_threads(bytes, [&]() { return hipSetDevice(c->device) == hipSuccess; }, f);
 }
 
-// fill(b0, b1) packs bytes [b0, b1) of the staging buffer; [from, end) of it go
-// to its device twin (`copy`) on the context's stream
+// bytes [b0, b1) of the staging buffer to its device twin, on the context's stream
+hipError_t send_range(cable_gpu_ctx *c, size_t b0, size_t b1) {
+  return hipMemcpyAsync(c->d_stage + b0, c->h_stage + b0, b1 - b0, hipMemcpyHostToDevice, c->stream);
+}
+
+// fill(b0, b1) packs bytes [b0, b1) of the staging buffer; `bytes` of it go to
+// its device twin (`copy`) on the context's stream
 template <class F>
-hipError_t stage_up(cable_gpu_ctx *c, size_t from, size_t end, bool copy, F &&fill) {
-  const size_t bytes = end - from, units = (bytes + XFER_UNIT - 1) / XFER_UNIT;
-  std::vector<std::atomic<size_t>> packed(units);
-  for (auto &u : packed) u = 0;
+hipError_t stage_up(cable_gpu_ctx *c, size_t bytes, bool copy, F &&fill) {
+  if (bytes <= staging::SMALL) {
+    fill(0, bytes);
+    return copy ? send_range(c, 0, bytes) : hipSuccess;
+  }
   std::atomic<int> err(hipSuccess);
-  on_threads(c, bytes, [&](size_t b0, size_t b1) {
-    const size_t u = b0 / XFER_UNIT, u0 = u * XFER_UNIT, u1 = std::min(bytes, u0 + XFER_UNIT);
-    fill(from + b0, from + b1);
-    if (packed[u].fetch_add(b1 - b0) + (b1 - b0) == u1 - u0 && copy) {
-      const hipError_t e = hipMemcpyAsync(c->d_stage + from + u0, c->h_stage + from + u0, u1 - u0, hipMemcpyHostToDevice,
-                                          c->stream);
-      if (e != hipSuccess) err = e;
-    }
-  });
+  staging::chunks_on_threads(
+      {{0, bytes}}, [&]() { return hipSetDevice(c->device) == hipSuccess; }, [](size_t) {},
+      [&](size_t, size_t b0, size_t b1) { fill(b0, b1); },
+      [&](size_t b0, size_t b1) {
+        if (const hipError_t e = copy ? send_range(c, b0, b1) : hipSuccess) err = e;
+      },
+      [](size_t) {});
   return (hipError_t)err.load();
 }
 
@@ -330,22 +334,22 @@ struct StageList {
     const void *host;
     size_t off, bytes;
   };
-  std::vector<Seg> segs;
+  Seg segs[12];
+  int n = 0;
   size_t from = 0, end = 0;
   // the array's offset
-  size_t add(const void *host, size_t n) {
+  size_t add(const void *host, size_t bytes) {
     const size_t off = end;
-    segs.push_back({host, off, n});
-    end += align_up(n);
+    segs[n++] = {host, off, bytes};
+    end += align_up(bytes);
     return off;
   }
-  hipError_t up(cable_gpu_ctx *c) const {
-    return stage_up(c, from, end, true, [&](size_t b0, size_t b1) {
-      for (const Seg &g : segs) {
-        const size_t l0 = std::max(b0, g.off), l1 = std::min(b1, g.off + g.bytes);
-        if (l0 < l1) memcpy(c->h_stage + l0, (const unsigned char *)g.host + (l0 - g.off), l1 - l0);
-      }
-    });
+  void pack(cable_gpu_ctx *c, size_t b0, size_t b1) const {
+    for (int k = 0; k < n; k++) {
+      const Seg &g = segs[k];
+      const size_t l0 = std::max(b0, g.off), l1 = std::min(b1, g.off + g.bytes);
+      if (l0 < l1) memcpy(c->h_stage + l0, (const unsigned char *)g.host + (l0 - g.off), l1 - l0);
+    }
   }
 };
 
@@ -448,7 +452,7 @@ int batched_transfer(cable_gpu_ctx *c, int n, const int *ids, void *const *hosts
   const dim3 grid((unsigned)std::min<int64_t>(1024, (c->mp + 255) / 256), (unsigned)n);
   if (up) {
     c->touched = true;
-    const hipError_t e = stage_up(c, 0, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, true); });
+    const hipError_t e = stage_up(c, off, !direct, [&](size_t b0, size_t b1) { pack(b0, b1, true); });
     if (e != hipSuccess) {
       (void)hipStreamSynchronize(c->stream);
       return fail(CABLE_E_HIP, "%s: %s", who, hipGetErrorString(e));
@@ -1043,12 +1047,12 @@ __device__ inline R met_svp(R tk) {
 }
 
 // Half of a met window's staging buffer: bound by the host's copies into it, and
-// in a new context by the first touch of its pages (0.06 ms a MiB on eight
-// threads).  12 steps of 131,071 tiles (48 MiB) 1.2 ms, in a new context 3.4 ms;
-// in one buffer of up to 64 MiB 1.1 and 4.8 ms, in halves of 4 MiB 1.3 and 3.3,
-// of 16 MiB 1.2 and 4.5; in 13 buffers allocated and copied one by one
-// from pageable memory 2.0 and 8.0 ms (2.5 where the runtime had the memory of
-// closed contexts at hand, here 4.1).
+// in a new context by pinning it and by the first touch of its pages (0.06 ms a
+// MiB on eight threads) unless the runtime has a closed context's at hand.  12
+// steps of 131,071 tiles (48 MiB) 1.2 ms, in a new context 2.5 ms (2.2 to 4.7
+// where contexts had been closed before); in one buffer of up to 64 MiB 1.15, 4.5
+// and 2.1 to 7.4 ms, in halves of 4 MiB 1.3, 2.5 and 3.0; in 13 buffers
+// allocated and copied one by one from pageable memory 2.0, 8.0 and 2.5 to 4.4.
 constexpr size_t MET_STAGE = 8 << 20;
 
 struct MetArgs {
@@ -1106,6 +1110,30 @@ __global__ void __launch_bounds__(256) met_kernel(int64_t mp, MetArgs m, R *fsd1
   precip[o] = (R)m.rainf[src] * (R)m.rainf_scale;
   fld[o] = lw;
   coszen[o] = z;
+}
+
+// the kernel for steps s0 .. s0 + ns - 1 of a window, its variables at the offsets
+// `at` of the staging buffer
+hipError_t met_launch(cable_gpu_ctx *c, const cable_gpu_met *m, const size_t at[8], size_t lat, size_t elev, size_t hods,
+                      size_t doys, int s0, int ns) {
+  const float *const vars[8] = {m->swdown, m->lwdown, m->tair, m->qair, m->wind, m->wind_e, m->psurf, m->rainf};
+  auto var = [&](int v) { return vars[v] ? (const float *)(c->d_stage + at[v]) : nullptr; };
+  const MetArgs a = {var(0), var(1), var(2), var(3), var(4), var(5), var(6), var(7), c->d_order,
+                     m->elevation ? (const double *)(c->d_stage + elev) : nullptr,
+                     (const double *)(c->d_stage + lat), (const double *)(c->d_stage + hods) + s0,
+                     (const double *)(c->d_stage + doys) + s0, m->tair_offset, m->psurf_scale, m->rainf_scale,
+                     m->qair_is_rh};
+  const dim3 grid((unsigned)((c->mp + 255) / 256), (unsigned)ns);
+  auto go = [&](auto zero) {
+    using R = decltype(zero);
+    R *f[8];
+    for (int i = 0; i < 8; i++) f[i] = (R *)c->forc[i] + (size_t)s0 * (size_t)c->mp;
+    hipLaunchKernelGGL(met_kernel<R>, grid, dim3(256), 0, c->stream, c->mp, a, f[0], f[1], f[2], f[3], f[4], f[5],
+                       f[6], f[7]);
+  };
+  if (c->precision == CABLE_PREC_MIXED) go(0.0f);
+  else go(0.0);
+  return hipGetLastError();
 }
 
 // the reader's clock (src/offline/cable_input.F90:1685-1850, local time):
@@ -1297,7 +1325,7 @@ int cable_gpu_synth_forcing(cable_gpu_ctx *c, int k_first, int nsteps, uint64_t 
   in.add(t0, sizeof(double) * mp);
   const size_t lat_off = in.add(lat, sizeof(double) * mp);
   if (const int r = ensure_stage(c, in.end)) return r;
-  const hipError_t e = in.up(c);
+  const hipError_t e = stage_up(c, in.end, true, [&](size_t b0, size_t b1) { in.pack(c, b0, b1); });
   if (e != hipSuccess) {
     (void)hipStreamSynchronize(c->stream);
     return fail(CABLE_E_HIP, "cable_gpu_synth_forcing: %s", hipGetErrorString(e));
@@ -1354,9 +1382,9 @@ int cable_gpu_set_met(cable_gpu_ctx *c, int k_first, int nsteps, double dels, co
     for (int i = 0; i < 8; i++) HIPCHECK(hipMalloc(&c->forc[i], bytes));
   }
   // the met variables to the device in the caller's tile order, through the
-  // staging buffer: what does not change with the steps, then the steps in
-  // chunks through the buffer's two halves in turn, so that the host packs one
-  // while the other is copied
+  // staging buffer: what does not change with the steps, and the steps in chunks
+  // through the buffer's two halves in turn, so that the host packs one while
+  // the other is copied
   const float *const vars[8] = {m->swdown, m->lwdown, m->tair, m->qair, m->wind, m->wind_e, m->psurf, m->rainf};
   size_t per_step = 0;
   for (const float *v : vars) per_step += v ? sizeof(float) * mp : 0;
@@ -1368,42 +1396,53 @@ int cable_gpu_set_met(cable_gpu_ctx *c, int k_first, int nsteps, double dels, co
   const size_t doys = fixed.add(doy.data(), sizeof(double) * doy.size());
   size_t half = 0;
   for (const float *v : vars) half += v ? align_up(sizeof(float) * (size_t)chunk * mp) : 0;
-  if (const int r = ensure_stage(c, fixed.end + (chunk < nsteps ? 2 : 1) * half)) return r;
-  c->nsteps_forc = 0;  // the window there is overwritten from here on
-  hipError_t e = ensure_events(c, 2);
-  if (e == hipSuccess) e = fixed.up(c);
-  for (int s0 = 0, q = 0; s0 < nsteps && e == hipSuccess; s0 += chunk, q++) {
-    const int ns = std::min(chunk, nsteps - s0);
-    StageList in;
-    in.from = in.end = fixed.end + (size_t)(q & 1) * half;
-    size_t at[8];
+  // a chunk's arrays, the first with what does not change in front
+  auto steps_of = [&](size_t q) { return std::min(chunk, nsteps - (int)q * chunk); };
+  auto list = [&](size_t q, size_t at[8]) {
+    StageList in = q ? StageList() : fixed;
+    if (q) in.from = in.end = fixed.end + (q & 1) * half;
     for (int v = 0; v < 8; v++)
-      at[v] = vars[v] ? in.add(vars[v] + (size_t)s0 * mp, sizeof(float) * (size_t)ns * mp) : 0;
-    if (q > 1) e = hipEventSynchronize(c->xev[q & 1]);
-    if (e == hipSuccess) e = in.up(c);
-    if (e == hipSuccess) e = hipEventRecord(c->xev[q & 1], c->stream);
-    if (e != hipSuccess) break;
-    auto var = [&](int v) { return vars[v] ? (const float *)(c->d_stage + at[v]) : nullptr; };
-    const MetArgs a = {var(0), var(1), var(2), var(3), var(4), var(5), var(6), var(7), c->d_order,
-                       m->elevation ? (const double *)(c->d_stage + elev) : nullptr,
-                       (const double *)(c->d_stage + lat), (const double *)(c->d_stage + hods) + s0,
-                       (const double *)(c->d_stage + doys) + s0, m->tair_offset, m->psurf_scale, m->rainf_scale,
-                       m->qair_is_rh};
-    const dim3 grid((unsigned)((mp + 255) / 256), (unsigned)ns);
-    auto go = [&](auto zero) {
-      using R = decltype(zero);
-      R *f[8];
-      for (int i = 0; i < 8; i++) f[i] = (R *)c->forc[i] + (size_t)s0 * mp;
-      hipLaunchKernelGGL(met_kernel<R>, grid, dim3(256), 0, c->stream, c->mp, a, f[0], f[1], f[2], f[3], f[4], f[5],
-                         f[6], f[7]);
-    };
-    if (c->precision == CABLE_PREC_MIXED) go(0.0f);
-    else go(0.0);
-    e = hipGetLastError();
+      at[v] = vars[v] ? in.add(vars[v] + q * chunk * mp, sizeof(float) * (size_t)steps_of(q) * mp) : 0;
+    return in;
+  };
+  std::vector<staging::Range> chunks;
+  for (size_t q = 0; (int)q * chunk < nsteps; q++) {
+    size_t at[8];
+    const StageList in = list(q, at);
+    chunks.push_back({in.from, in.end});
   }
+  if (const int r = ensure_stage(c, fixed.end + std::min<size_t>(2, chunks.size()) * half)) return r;
+  std::atomic<int> err((int)ensure_events(c, 2));
+  auto check = [&](hipError_t e) {
+    if (e != hipSuccess) err = e;
+  };
+  c->nsteps_forc = 0;  // the window there is overwritten from here on
+  std::atomic<size_t> closed[2] = {{0}, {0}};  // chunks of a half whose copies are queued
+  staging::chunks_on_threads(
+      chunks, [&]() { return hipSetDevice(c->device) == hipSuccess; },
+      [&](size_t q) {  // the half's last chunk has left the host's side of it
+        if (q < 2) return;
+        while (closed[q & 1] < q / 2) std::this_thread::yield();
+        if (err == hipSuccess) check(hipEventSynchronize(c->xev[q & 1]));
+      },
+      [&](size_t q, size_t b0, size_t b1) {
+        size_t at[8];
+        list(q, at).pack(c, b0, b1);
+      },
+      [&](size_t b0, size_t b1) {
+        if (err == hipSuccess) check(send_range(c, b0, b1));
+      },
+      [&](size_t q) {
+        size_t at[8];
+        list(q, at);
+        if (err == hipSuccess) check(hipEventRecord(c->xev[q & 1], c->stream));
+        if (err == hipSuccess) check(met_launch(c, m, at, lat, elev, hods, doys, (int)q * chunk, steps_of(q)));
+        closed[q & 1]++;
+      });
   const hipError_t w = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) e = w;
-  if (e != hipSuccess) return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString(e));
+  if (err == hipSuccess) check(w);
+  if (err != hipSuccess)
+    return fail(CABLE_E_HIP, "cable_gpu_set_met: %s", hipGetErrorString((hipError_t)err.load()));
   const int ids[8] = {CABLE_F_met_fsd, CABLE_F_met_fld, CABLE_F_met_tk, CABLE_F_met_qv,
                       CABLE_F_met_ua, CABLE_F_met_pmb, CABLE_F_met_precip, CABLE_F_met_coszen};
   std::vector<void *> tab = c->dev;

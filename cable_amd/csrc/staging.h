@@ -66,18 +66,17 @@ struct Pieces {
   constexpr size_t count() const { return large + (bytes - large * LARGE + SMALL - 1) / SMALL; }
 };
 
-// f(b0, b1) for every piece [b0, b1) of `bytes`; init() on each thread that is
-// started, which takes no piece if it is false
+// f(q) for every q below `count`, claimed in order by the threads that `bytes` of
+// work ask for; init() on each thread that is started, which claims none if it
+// is false
 template <class Init, class F>
-void on_threads(size_t bytes, Init &&init, F &&f) {
-  const Pieces p(bytes);
-  const size_t pieces = p.count();
+void share_out(size_t bytes, size_t count, Init &&init, F &&f) {
   std::atomic<size_t> next(0);
   auto run = [&]() {
-    for (size_t q; (q = next.fetch_add(1)) < pieces;) f(p.begin(q), p.begin(q + 1));
+    for (size_t q; (q = next.fetch_add(1)) < count;) f(q);
   };
   const unsigned nt = (unsigned)std::min<size_t>(
-      {THREADS, pieces, bytes / PER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
+      {THREADS, count, bytes / PER_THREAD + 1, std::max(1u, std::thread::hardware_concurrency())});
   std::vector<std::thread> th;
   for (unsigned t = 1; t < nt; t++) {
     try {
@@ -90,6 +89,53 @@ void on_threads(size_t bytes, Init &&init, F &&f) {
   }
   run();
   for (auto &t : th) t.join();
+}
+
+// f(b0, b1) for every piece [b0, b1) of `bytes`
+template <class Init, class F>
+void on_threads(size_t bytes, Init &&init, F &&f) {
+  const Pieces p(bytes);
+  share_out(bytes, p.count(), init, [&](size_t q) { f(p.begin(q), p.begin(q + 1)); });
+}
+
+// Chunks of a buffer that is smaller than what goes through it: chunk q is packed
+// when release(q) has returned, sent unit by unit when its parts are packed and
+// closed by the thread that sent its last unit.  Chunks are begun in order, so
+// that release(q) may wait for the closing of an earlier one.
+struct Range {
+  size_t from, end;
+};
+template <class Init, class Release, class Fill, class Send, class Close>
+void chunks_on_threads(const std::vector<Range> &chunks, Init &&init, Release &&release, Fill &&fill, Send &&send,
+                       Close &&close) {
+  struct Part {
+    size_t chunk, b0, b1, unit, of;  // bytes [b0, b1) of unit `unit`, of which there are `of`
+  };
+  std::vector<Part> parts;
+  size_t units = 0, total = 0;
+  for (size_t q = 0; q < chunks.size(); q++) {
+    const size_t bytes = chunks[q].end - chunks[q].from;
+    const Pieces p(bytes);
+    for (size_t k = 0; k < p.count(); k++) {
+      const size_t b0 = p.begin(k), u0 = b0 / UNIT * UNIT;
+      parts.push_back({q, b0, p.begin(k + 1), units + b0 / UNIT, std::min(bytes, u0 + UNIT) - u0});
+    }
+    units += (bytes + UNIT - 1) / UNIT;
+    total += bytes;
+  }
+  std::vector<std::atomic<size_t>> packed(units), sent(chunks.size());
+  for (auto &x : packed) x = 0;
+  for (auto &x : sent) x = 0;
+  share_out(total, parts.size(), init, [&](size_t k) {
+    const Part &t = parts[k];
+    const Range &r = chunks[t.chunk];
+    release(t.chunk);
+    fill(t.chunk, r.from + t.b0, r.from + t.b1);
+    if (packed[t.unit].fetch_add(t.b1 - t.b0) + (t.b1 - t.b0) != t.of) return;
+    const size_t u0 = r.from + t.b0 / UNIT * UNIT;
+    send(u0, u0 + t.of);
+    if (sent[t.chunk].fetch_add(t.of) + t.of == r.end - r.from) close(t.chunk);
+  });
 }
 
 }  // namespace staging

@@ -35,5 +35,22 @@ def test_a_large_buffer_is_not_shared_within_a_huge_page(lines):
     assert all(most == 1 for k, v in lines if k == "pieces" for most in v[3:])
 
 
+def test_chunks_through_two_halves(lines):
+    """Each closed once and in its half's turn, and all bytes arrive."""
+    got = [v for k, v in lines if k == "chunks"]
+    assert len(got) == 3 and all(n == 11 and closed == 11 and early == 0 and same for n, closed, early, same in got)
+
+
+def test_no_data_race(tmp_path):
+    """The same program under the thread sanitizer."""
+    exe = str(tmp_path / "s")
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=thread", "-pthread",
+                        os.path.join(HERE, "host_staging.cpp"), "-o", exe], capture_output=True, text=True)
+    if r.returncode != 0:
+        pytest.skip("sanitizer build unavailable: " + r.stderr[-300:])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "WARNING: ThreadSanitizer" not in r.stderr, r.stderr[-3000:]
+
+
 def test_a_small_context_pins_once(lines):
     assert [v for k, v in lines if k == "pins"] == [[77, 1], [1000, 1], [4093, 2], [20011, 2]]
