@@ -263,8 +263,9 @@ struct LateStage {
 // loaded (again) after the canopy; FIELD_SETTLED: the radiation, roughness and
 // air diagnostics, written before the leaf iteration; FIELD_CANOPY: the
 // canopy's, written after it.  The rest is scattered at the end.  Scratch 1,424
-// -> 480 B per lane (FP64); a step of 262,144 tiles 1.08 -> 0.75 ms (0.96 GB,
-// 1.3 TB/s), of 77 tiles 171 -> 150 us.
+// -> 480 B per lane (FP64; 216 B without hoisting in machine loops, as it is built
+// now); a step of 262,144 tiles 1.08 -> 0.75 ms (0.96 GB, 1.3 TB/s; 0.68 as built
+// now), of 77 tiles 171 -> 150 us.
 enum { FIELD_LATE_ONLY = 1, FIELD_RELOAD = 2, FIELD_LATE = 3, FIELD_SETTLED = 4, FIELD_CANOPY = 8 };
 constexpr int field_phase(int id) {
   switch (id) {
@@ -1054,7 +1055,7 @@ __global__ void __launch_bounds__(64 * NWAVES) mlp_infer_kernel(StepArgs a, cons
 }
 
 
-// launch one step over mp tiles on `stream` (256 threads per workgroup)
+// launch the step (or a.nsteps plain resident ones) over mp tiles on `stream`
 template <class R, bool FULL, bool TABLES, int MODE = MODE_PLAIN, bool CONS = false>
 hipError_t launch_cbm(const StepArgs &a, int64_t mp, hipStream_t stream) {
   // FP64 runs one wave per SIMD: one-wave workgroups let the dispatcher fill
